@@ -1,6 +1,9 @@
-// A1 camera rays, A2 tile DDA, and the one-thread-per-ray FP32 renderer (the plain path).
+// A1 camera rays, A2 tile DDA, and the plain FP32 renderer (march, FP32 MFMA MLP and compositing in one
+// kernel, no workspace).
+#include "mfma_ops.hpp"
 #include "snisr_common.hpp"
 #include "snisr_device.hpp"
+#include "train_mma.hpp"
 
 namespace snisr {
 
@@ -85,49 +88,249 @@ __global__ void k_pack_f32t(const float* __restrict__ src, int64_t src_stride, f
 }
 
 // ---------------------------------------------------------------------------- FP32 render
-template <int F, int WD, int L, bool HALF>
-__global__ __launch_bounds__(64) void k_render_fp32(snisr_scene S, snisr_march_params P, snisr_rays R,
-                                                    snisr_render_out O, int packet_w) {
-  constexpr int IN = F + 15;
-  constexpr int XD = IN > WD ? IN : WD;
-  __shared__ float lds[XD * 64];
-  float* xs = lds + threadIdx.x;
-  const int64_t tid = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (tid >= R.n) return;
-  const int64_t i = ray_of_thread(tid, R.n, packet_w);
-  const float* og = R.origins + i * R.origin_stride;
-  const V3 origin = v3(og[0], og[1], og[2]);
-  const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
-  const float t_hit = R.t_hit ? R.t_hit[i] : __builtin_inff();
-  float enc[15];
-  view_encoding(d, enc);
-  constexpr int64_t wstride = f32t_stride(IN, WD, L);
-  float col[3] = {0.0f, 0.0f, 0.0f};
-  int32_t* bricks = O.bricks ? O.bricks + i * O.brick_cap : nullptr;
-  MarchResult res;
-  march_ray(S, P, origin, d, t_hit, R.visited ? R.visited + i * P.max_tiles : nullptr, bricks, O.brick_cap,
-            [&](int tile, const V3&, const Corners& c, float w, float, float, float) {
-              gather_features<F, HALF>(S.feats, c, xs);
+// One wavefront takes 64 / kFp32Group rays, marched by groups of kFp32Group lanes (GroupMarch), and
+// queues every sample's record in LDS; whenever 64 records are queued it evaluates their MLP together as
+// the columns of v_mfma_f32_32x32x2_f32 products (activations in registers: the D layout of a layer is
+// the B operand of the next, the weights read from the f32t packing, whose rows are the A operand's
+// columns) and adds the weighted colours to their rays in sample order.
+//
+// What bounds it: the matrix products (12.5 kFLOP per sample at width 64).  The previous form ran one
+// ray and one sample's MLP per lane on the vector units, re-reading every weight per sample and leaving
+// most lanes idle once their rays had ended: 11.8 ms for the 320x180 single-tile view, 0.21 ms now; 85 ms
+// for the 1280x720 frame of the 16-tile room, 10.1 ms now.  Eight lanes per ray: with 4 the small view takes
+// 0.25 ms and the room 10.2, with 16 0.25 and 10.7 (more of the lanes past a brick's or ray's end).
+constexpr int kFp32Group = 8, kFp32Rays = 64 / kFp32Group;
+
+// acc += the product of one layer's f32t weights Wt[in][OUT4] with x over NS steps, all output blocks
+// at once (consecutive products are independent); rows past the layer's ROWS inputs count as zero
+template <int NS, int ROWS, int NOB, int CB, int OUT4>
+__device__ __forceinline__ void f32t_product(const float* __restrict__ Wt, const float (*x)[64], int c, int h,
+                                             f32x16 (&acc)[CB][NOB]) {
+  constexpr int GS = 4;  // steps whose weights are loaded together, one such group ahead of the products
+  float a[2][GS][NOB];
+  // the lane's offset is hidden from the optimizer: the loads' addresses would otherwise be formed
+  // once, outside the march loop, and held in registers
+  int off = 4 * h * OUT4 + (c < OUT4 ? c : 0);
+  asm volatile("" : "+v"(off));
+  auto fetch = [&](int g, float (&v)[GS][NOB]) {
 #pragma unroll
-              for (int k = 0; k < 15; ++k) xs[(F + k) * 64] = enc[k];
-              float rgb[3];
-              const int t0 = __builtin_amdgcn_readfirstlane(tile);
-              if (__all(tile == t0)) mlp_f32<IN, WD, L>(S.mlp_f32t + (int64_t)t0 * wstride, xs, rgb);
-              else mlp_f32<IN, WD, L>(S.mlp_f32t + (int64_t)tile * wstride, xs, rgb);
+    for (int q = 0; q < GS; ++q)
 #pragma unroll
-              for (int ch = 0; ch < 3; ++ch) col[ch] = col[ch] + w * rgb[ch];
-            },
-            res);
-  if (bricks)
-    for (int k = res.n_bricks; k < O.brick_cap; ++k) bricks[k] = -1;
-  if (O.rgb) {
-    O.rgb[3 * i] = col[0];
-    O.rgb[3 * i + 1] = col[1];
-    O.rgb[3 * i + 2] = col[2];
+      for (int ob = 0; ob < NOB; ++ob) {
+        const float w = Wt[tr_row(g * GS + q, 0) * OUT4 + ob * 32 + off];
+        const bool row_ok = tr_row(g * GS + q, 1) < ROWS || h == 0;  // lane half 1 holds the row 4 further on
+        v[q][ob] = c < OUT4 && row_ok ? w : 0.0f;
+      }
+  };
+  fetch(0, a[0]);
+#pragma unroll
+  for (int g = 0; g < NS / GS; ++g) {
+    if (g + 1 < NS / GS) fetch(g + 1, a[(g + 1) & 1]);
+#pragma unroll
+    for (int q = 0; q < GS; ++q)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int ob = 0; ob < NOB; ++ob)
+          acc[cb][ob] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g & 1][q][ob], x[cb][g * GS + q], acc[cb][ob], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  if (O.T) O.T[i] = res.T;
-  if (O.n_samples) O.n_samples[i] = res.n_samples;
-  if (O.depth) O.depth[i] = res.depth;
+}
+
+// out = b (in the D layout) for NOB blocks of CB column blocks
+template <int NOB, int CB>
+__device__ __forceinline__ void f32t_bias(const float* __restrict__ b, int h, f32x16 (&acc)[CB][NOB]) {
+#pragma unroll
+  for (int ob = 0; ob < NOB; ++ob)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 v = *reinterpret_cast<const float4*>(b + 32 * ob + 8 * q + 4 * h);
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) {
+        acc[cb][ob][4 * q] = v.x;
+        acc[cb][ob][4 * q + 1] = v.y;
+        acc[cb][ob][4 * q + 2] = v.z;
+        acc[cb][ob][4 * q + 3] = v.w;
+      }
+    }
+}
+
+// The MLP of CB blocks of 32 columns in one tile: x[cb] the layer-0 inputs in step order (overwritten),
+// z[cb][0..2] the output pre-activations (lanes of half 0)
+template <int IN, int WD, int L, int CB>
+__device__ __forceinline__ void f32t_mlp(const float* __restrict__ P, float (*x)[64], int c, int h, float (*z)[3]) {
+  constexpr int NOB = WD / 32;
+  auto relu_into = [&](f32x16(&acc)[CB][NOB]) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int r = 0; r < 16 * NOB; ++r) x[cb][r] = acc[cb][r / 16][r % 16] > 0.0f ? acc[cb][r / 16][r % 16] : 0.0f;
+  };
+  {
+    f32x16 acc[CB][NOB];
+    f32t_bias<NOB, CB>(P + IN * WD, h, acc);
+    f32t_product<tr_ns0(IN), IN, NOB, CB, WD>(P, x, c, h, acc);
+    relu_into(acc);
+  }
+  P += IN * WD + WD;
+#pragma unroll 1
+  for (int l = 1; l < L - 1; ++l) {
+    f32x16 acc[CB][NOB];
+    f32t_bias<NOB, CB>(P + WD * WD, h, acc);
+    f32t_product<WD / 2, WD, NOB, CB, WD>(P, x, c, h, acc);
+    relu_into(acc);
+    P += WD * WD + WD;
+  }
+  f32x16 acc[CB][1];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) acc[cb][0] = f32x16{};
+  f32t_product<WD / 2, WD, 1, CB, 4>(P, x, c, h, acc);
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) z[cb][i] = acc[cb][0][i] + P[WD * 4 + i];
+}
+
+// two waves per SIMD at least: one wave's march waits while the other's products run
+template <int F, int WD, int L, bool HALF>
+__global__ __launch_bounds__(64, 2) void k_render_fp32(snisr_scene S, snisr_march_params P, snisr_rays R,
+                                                    snisr_render_out O, int packet_w) {
+  constexpr int G = kFp32Group, RPW = 64 / G, IN = F + 15, NS0 = tr_ns0(IN), QCAP = 128;
+  constexpr int CB = WD <= 64 ? 2 : 1;  // column blocks per pass of the MLP (registers at width 128)
+  static_assert(WD % 32 == 0 && WD <= 128 && F % 8 == 0 && F <= 32 && NS0 <= 64, "MLP shape");
+  __shared__ float4 q_rec[QCAP];        // voxel coordinate, compositing weight
+  __shared__ int q_tile[QCAP], q_ray[QCAP];
+  __shared__ float enc_lds[RPW][17];
+  __shared__ float res[64][3];          // weighted colours of the batch
+  const int lane = threadIdx.x, c = lane & 31, h = lane >> 5;
+  const int rl = lane / G;              // this lane's ray within the wavefront
+  const int64_t tid = (int64_t)blockIdx.x * RPW + rl;
+  constexpr int64_t wstride = f32t_stride(IN, WD, L);
+  const bool has = tid < R.n;
+  const int64_t i = has ? ray_of_thread(tid, R.n, packet_w) : 0;
+  GroupMarch<G> m;
+  m.phase = GroupMarch<G>::kDone;
+  int32_t* bricks = has && O.bricks ? O.bricks + i * O.brick_cap : nullptr;
+  if (has) {
+    const float* og = R.origins + i * R.origin_stride;
+    const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
+    m.init(S, P, v3(og[0], og[1], og[2]), d, R.t_hit ? R.t_hit[i] : __builtin_inff(),
+           R.visited ? R.visited + i * P.max_tiles : nullptr);
+    if (lane % G == 0) {
+      float enc[15];
+      view_encoding(d, enc);
+#pragma unroll
+      for (int k = 0; k < 15; ++k) enc_lds[rl][k] = enc[k];
+    }
+  }
+  // lane 3 r + ch < 3 RPW sums channel ch of ray r
+  float col = 0.0f;
+  int qn = 0;  // queued records (wave-uniform)
+  auto sync = [&] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // evaluates the first nq <= 64 queued records and adds their colours
+  auto shade = [&](int nq) {
+    sync();
+    uint64_t todo = nq >= 64 ? ~0ull : (1ull << nq) - 1;
+    const int own_tile = lane < nq ? q_tile[lane] : -1;
+    // one pass per distinct tile among the records (nearly always one)
+    while (todo) {
+      const int t = __builtin_amdgcn_readlane(own_tile, __builtin_ctzll(todo));
+      const uint64_t in_t = __builtin_amdgcn_ballot_w64(own_tile == t);
+      todo &= ~in_t;
+#pragma unroll 1
+      for (int c0 = 0; c0 < 2; c0 += CB) {
+        if (!((in_t >> (32 * c0)) & (CB == 2 ? ~0ull : 0xffffffffull))) continue;
+        float x[CB][64];
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          const int r = 32 * (c0 + cb) + c;
+          const bool ok = in_t >> r & 1;
+          const float4 rec = ok ? q_rec[r] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          Corners cn;
+          find_corners(S.brick_map + S.tile_brick_base[t], S.tile_res[t], v3(rec.x, rec.y, rec.z), cn);
+          uint32_t mask[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) mask[k] = corner_mask(ok && cn.slot[k] >= 0);
+          gather_rows<F, HALF>(S.feats, cn, mask, h, x[cb]);
+          __builtin_amdgcn_sched_barrier(0);  // one block's corner rows in registers at a time
+          const float* e = enc_lds[ok ? q_ray[r] : 0];
+#pragma unroll
+          for (int s = 0; s < NS0; ++s) {
+            const int r0 = tr_row(s, 0) - F, r1 = tr_row(s, 1) - F;  // encoding entry of each half
+            if (r0 >= 0) x[cb][s] = h ? (r1 < 15 ? e[r1 < 15 ? r1 : 0] : 0.0f) : (r0 < 15 ? e[r0 < 15 ? r0 : 0] : 0.0f);
+          }
+        }
+        float z[CB][3];
+        f32t_mlp<IN, WD, L, CB>(S.mlp_f32t + (int64_t)t * wstride, x, c, h, z);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          const int r = 32 * (c0 + cb) + c;
+          if (h == 0 && (in_t >> r & 1)) {
+            const float w = q_rec[r].w;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) res[r][k] = w * sigmoid_cw(z[cb][k]);
+          }
+        }
+      }
+    }
+    sync();
+    if (lane < 3 * RPW) {
+      const int ray = lane / 3, ch = lane - 3 * ray;
+      for (int r = 0; r < nq; ++r)
+        if (q_ray[r] == ray) col = col + res[r][ch];
+    }
+    sync();
+  };
+  while (true) {
+    const bool live = m.phase != GroupMarch<G>::kDone;
+    const bool marching = __builtin_amdgcn_ballot_w64(live) != 0;
+    if (!marching && qn == 0) break;
+    float4 rec;
+    int tile = 0;
+    bool took = false;
+    if (live) {
+      const bool turn = tile_quorum(m.phase == GroupMarch<G>::kTile);
+      took = m.step(S, P, turn, bricks, O.brick_cap,
+                    [&](int t, const V3& f, const Corners&, float w, float, float, float, int) {
+                      rec = make_float4(f.x, f.y, f.z, w);
+                      tile = t;
+                    });
+    }
+    // a ray's samples of one step sit on consecutive lanes, so the queue keeps every ray's order
+    const uint64_t tm = __builtin_amdgcn_ballot_w64(took);
+    if (took) {
+      const int at = qn + __builtin_popcountll(tm & ((1ull << lane) - 1));
+      q_rec[at] = rec;
+      q_tile[at] = tile;
+      q_ray[at] = rl;
+    }
+    qn += __builtin_popcountll(tm);
+    if (qn >= 64 || !marching) {  // a full batch, or what is left at the end
+      const int nq = qn < 64 ? qn : 64;
+      shade(nq);
+      qn -= nq;
+      if (lane < qn) {  // fewer than 64 remain: they move to the front
+        q_rec[lane] = q_rec[64 + lane];
+        q_tile[lane] = q_tile[64 + lane];
+        q_ray[lane] = q_ray[64 + lane];
+      }
+    }
+  }
+  if (has && lane % G == 0) {
+    if (bricks)
+      for (int k = m.nbr; k < O.brick_cap; ++k) bricks[k] = -1;
+    if (O.T) O.T[i] = m.T;
+    if (O.n_samples) O.n_samples[i] = m.nsamp;
+    if (O.depth) O.depth[i] = m.depth;
+  }
+  if (lane < 3 * RPW) {
+    const int64_t t = (int64_t)blockIdx.x * RPW + lane / 3;
+    if (t < R.n) O.rgb[3 * ray_of_thread(t, R.n, packet_w) + lane % 3] = col;
+  }
 }
 
 // sigma-only march (no MLP): counts, T, depth, bricks; used when rgb is not requested.
@@ -224,7 +427,8 @@ int snisr_render_fp32(const snisr_scene* scene, const snisr_march_params* params
 #define SNISR_FP32_CASE(F_, W_, L_, H_)                                                                   \
   if (F == F_ && WD == W_ && L == L_ && half == H_) {                                                     \
     SNISR_HIP(stage_event(out, 0, st));                                                                   \
-    hipLaunchKernelGGL((k_render_fp32<F_, W_, L_, H_>), grid, dim3(64), 0, st, *scene, *params, *rays, *out, pw); \
+    hipLaunchKernelGGL((k_render_fp32<F_, W_, L_, H_>), dim3((unsigned)((rays->n + kFp32Rays - 1) / kFp32Rays)), \
+                       dim3(64), 0, st, *scene, *params, *rays, *out, pw);                                \
     SNISR_LAUNCHED();                                                                                     \
     SNISR_HIP(stage_event(out, 1, st));                                                                   \
     return SNISR_OK;                                                                                      \

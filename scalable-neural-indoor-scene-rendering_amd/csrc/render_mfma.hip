@@ -1475,41 +1475,16 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
     view_encoding(d, enc);
   }
   float x0[NS0];
+  gather_rows<F, HALF>(S.feats, cn, cmask, h, x0);
 #pragma unroll
-  for (int g = 0; g < NS0 / 4; ++g) {
+  for (int g = F / 8; g < NS0 / 4; ++g) {
     const int base = 32 * (g / 4) + 8 * (g % 4);  // first row of the 8-row group (lane half 0)
-    if (base < F) {
-      float v[8][4];
 #pragma unroll
-      // unconditional loads (empty corners read slot 0, which exists whenever a lane of the
-      // chunk is valid, and are zeroed after), so the eight loads are in flight together
-      for (int q = 0; q < 8; ++q) {
-        const int64_t off = (int64_t)(cn.slot[q] >= 0 ? cn.slot[q] : 0) * F + base + 4 * h;
-        const uint32_t m = cmask[q];
-        if (HALF) {
-          uint2 raw = *reinterpret_cast<const uint2*>(reinterpret_cast<const _Float16*>(S.feats) + off);
-          raw.x &= m;
-          raw.y &= m;
-          const _Float16* hv = reinterpret_cast<const _Float16*>(&raw);
-#pragma unroll
-          for (int t = 0; t < 4; ++t) v[q][t] = (float)hv[t];
-        } else {
-          FeatLoad<false>::load(S.feats, off, m, v[q]);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float qv[8] = {v[0][t], v[1][t], v[2][t], v[3][t], v[4][t], v[5][t], v[6][t], v[7][t]};
-        x0[4 * g + t] = tri_combine(qv, cn.wx, cn.wy, cn.wz);
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int e0 = base - F + t, e1 = e0 + 4;  // view-encoding index for lane half 0 / 1
-        const float v0 = e0 < 15 ? enc[e0 < 15 ? e0 : 0] : 0.0f;
-        const float v1 = e1 < 15 ? enc[e1 < 15 ? e1 : 0] : 0.0f;
-        x0[4 * g + t] = h ? v1 : v0;
-      }
+    for (int t = 0; t < 4; ++t) {
+      const int e0 = base - F + t, e1 = e0 + 4;  // view-encoding index for lane half 0 / 1
+      const float v0 = e0 < 15 ? enc[e0 < 15 ? e0 : 0] : 0.0f;
+      const float v1 = e1 < 15 ? enc[e1 < 15 ? e1 : 0] : 0.0f;
+      x0[4 * g + t] = h ? v1 : v0;
     }
   }
   const float* P = W.frag + (int64_t)tile * STRIDE;

@@ -491,6 +491,194 @@ struct FlatMarch {
   }
 };
 
+// One ray per group of G consecutive lanes (G divides 64).  A wavefront that marches one ray per lane
+// waits for one brick-table load per empty cell and one density gather per sample; a launch of few
+// rays has too few wavefronts to cover those waits.  Here the lanes of a group look ahead together:
+// lane g tests the cell g steps further along the brick walk, and in an occupied brick lane g
+// evaluates sample k + g, so one memory round trip serves G cells or samples.  Every lane of the
+// group keeps the same ray state; the transmittance is the same left-to-right product as in
+// march_ray (lane g multiplies the factors of lanes 0..g-1 in order), so cells, samples, T, depth and
+// counts are bit-identical to it.
+template <int G>
+struct GroupMarch {
+  enum { kTile, kWalk, kSample, kDone };
+  TileWalker walker;
+  V3 origin, d, o;
+  float t_hit, T, depth, tl, inv_vs, near_, far_;
+  const int32_t* vis;
+  const int32_t* bmap;
+  int nsamp, nbr, vi, tile, n, nb, k, phase;
+  bool first_hit;
+  int cur[3], stp[3];
+  float tmax[3], tdel[3];
+
+  __device__ __forceinline__ void init(const snisr_scene& S, const snisr_march_params& P, V3 origin_, V3 d_,
+                                       float t_hit_, const int32_t* __restrict__ vis_) {
+    origin = origin_;
+    d = d_;
+    t_hit = t_hit_;
+    vis = vis_;
+    if (!vis) walker.init(S, origin, d, P.max_tiles);
+    T = 1.0f;
+    nsamp = nbr = vi = n = nb = k = 0;
+    tile = -1;
+    depth = -1.0f;
+    first_hit = false;
+    tl = inv_vs = near_ = far_ = 0.0f;
+    o = v3(0.0f, 0.0f, 0.0f);
+    bmap = nullptr;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      cur[a] = 0;
+      stp[a] = 1;
+      tmax[a] = tdel[a] = 0.0f;
+    }
+    phase = kTile;
+  }
+  __device__ __forceinline__ void dda_step() {
+    int a;
+    if (tmax[0] < tmax[1]) a = (tmax[0] < tmax[2]) ? 0 : 2;
+    else a = (tmax[1] < tmax[2]) ? 1 : 2;
+    if (a == 0) { cur[0] += stp[0]; tmax[0] += tdel[0]; }
+    else if (a == 1) { cur[1] += stp[1]; tmax[1] += tdel[1]; }
+    else { cur[2] += stp[2]; tmax[2] += tdel[2]; }
+    near_ = far_;
+    far_ = fminx(fminx(tmax[0], tmax[1]), tmax[2]);
+  }
+  __device__ __forceinline__ static uint32_t group_bits(bool v, int base) {
+    return (uint32_t)(__builtin_amdgcn_ballot_w64(v) >> base) & (uint32_t)((1ull << G) - 1);
+  }
+  // One unit of work of the group (its lanes are always in the same phase, so the lane exchanges below
+  // only read active lanes).  on_sample(tile, f, corners, w, sigma, interval, T_after, i) runs on the
+  // lanes that took a sample, i = its index along the ray; returns true on those lanes.
+  template <class OnSample>
+  __device__ __forceinline__ bool step(const snisr_scene& S, const snisr_march_params& P, bool tile_turn,
+                                       int32_t* bricks, int brick_cap, OnSample&& on_sample) {
+    const int lane = threadIdx.x & 63, g = lane % G, base = lane - g;
+    const float ts = S.tile_size;
+    const float hs = ts / 2.0f;
+    if (phase == kTile) {
+      if (!tile_turn) return false;
+      if (vi >= P.max_tiles) { phase = kDone; return false; }
+      const int t = vis ? vis[vi] : walker.next();
+      ++vi;
+      if (t == -1 || T < P.early_stop) { phase = kDone; return false; }
+      const V3 tc = v3(S.tile_centers[3 * t], S.tile_centers[3 * t + 1], S.tile_centers[3 * t + 2]);
+      float th;
+      ray_aabb(origin, d, tc, v3(hs, hs, hs), tl, th);
+      if (tl == -1.0f) return false;
+      tile = t;
+      const V3 corner = v3(tc.x - hs, tc.y - hs, tc.z - hs);
+      const float hi = ts - 0.00001f;
+      o = v3(origin.x + tl * d.x - corner.x, origin.y + tl * d.y - corner.y, origin.z + tl * d.z - corner.z);
+      o = v3(clampx(o.x, 0.0f, hi), clampx(o.y, 0.0f, hi), clampx(o.z, 0.0f, hi));
+      n = S.tile_res[tile];
+      nb = n >> 3;
+      const float bs = ts / (float)nb;
+      inv_vs = 1.0f / (ts / (float)n);
+      bmap = S.brick_map + S.tile_brick_base[tile];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const float oa = get(o, a), da = get(d, a);
+        cur[a] = (int)(oa / bs);
+        stp[a] = da >= 0.0f ? 1 : -1;
+        float nbd = (float)(cur[a] + stp[a]) * bs;
+        if (stp[a] < 0) nbd += bs;
+        tmax[a] = safe_div(nbd - oa, da);
+        tdel[a] = safe_div(bs * (float)stp[a], da);
+      }
+      near_ = 0.0f;
+      far_ = fminx(fminx(tmax[0], tmax[1]), tmax[2]);
+      phase = kWalk;
+    } else if (phase == kWalk) {
+      // lane g walks g cells ahead (a cell index that left the grid never comes back: every axis only
+      // moves one way), then the group moves to the first cell that is occupied or outside
+#pragma unroll
+      for (int j = 1; j < G; ++j)
+        if (g >= j) dda_step();
+      const bool in = (unsigned)cur[0] < (unsigned)nb && (unsigned)cur[1] < (unsigned)nb && (unsigned)cur[2] < (unsigned)nb;
+      const int b = in ? bmap[(cur[0] * nb + cur[1]) * nb + cur[2]] : -1;
+      const uint32_t out_m = group_bits(!in, base), occ_m = group_bits(b != -1, base);
+      const uint32_t any = out_m | occ_m;
+      const int f = any ? __builtin_ctz(any) : G - 1;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        cur[a] = __shfl(cur[a], base + f);
+        tmax[a] = __shfl(tmax[a], base + f);
+      }
+      near_ = __shfl(near_, base + f);
+      far_ = __shfl(far_, base + f);
+      if (!any) {
+        dda_step();
+      } else if (out_m >> f & 1) {
+        phase = kTile;
+      } else {
+        if (bricks && g == f && nbr < brick_cap) bricks[nbr] = b;
+        ++nbr;
+        k = 0;
+        phase = kSample;
+      }
+    } else if (phase == kSample) {
+      const float step = P.sample_step;
+      const float z = __builtin_fmaf((float)(k + g), step, near_);
+      const float tg = tl + z;
+      const bool live = z < far_;
+      // z grows along the lanes, so the live ones come first
+      const int nl = __builtin_popcount(group_bits(live, base));
+      const uint32_t hit_m = group_bits(live && tg >= t_hit, base);
+      const int cand = hit_m ? __builtin_ctz(hit_m) : nl;
+      const bool act = g < cand;
+      float alpha = 0.0f, om = 1.0f, sig = 0.0f, interval = 0.0f;
+      V3 f = v3(0.0f, 0.0f, 0.0f);
+      Corners c;
+      if (act) {
+        const V3 p = v3(o.x + z * d.x, o.y + z * d.y, o.z + z * d.z);
+        f = v3(p.x * inv_vs - 0.5f, p.y * inv_vs - 0.5f, p.z * inv_vs - 0.5f);
+        find_corners(bmap, n, f, c);
+        sig = tri_sigma(S.sigma, c);
+        sig = sig > 0.0f ? sig : 0.0f;
+        interval = fminx(step, far_ - z);
+        alpha = 1.0f - exp_cw(-(sig * interval));
+        om = 1.0f - alpha;
+      }
+      float t = T;  // transmittance before this lane's sample
+#pragma unroll
+      for (int j = 0; j < G - 1; ++j) {
+        const float oj = __shfl(om, base + j);
+        t = g > j ? t * oj : t;
+      }
+      const float T_next = t * om;
+      const uint32_t stop_m = group_bits(act && T_next < P.early_stop, base);
+      const int take = stop_m ? __builtin_ctz(stop_m) + 1 : cand;
+      const bool mine = g < take;
+      const uint32_t deep_m = group_bits(mine && t < P.trans_th, base);
+      if (!first_hit && deep_m) {
+        first_hit = true;
+        depth = __shfl(tg, base + __builtin_ctz(deep_m));
+      }
+      if (mine) on_sample(tile, f, c, alpha * t, sig, interval, T_next, nsamp + g);
+      if (take > 0) T = __shfl(T_next, base + take - 1);
+      nsamp += take;
+      if (stop_m || hit_m) {
+        phase = kDone;
+      } else if (nl < G) {
+        dda_step();
+        phase = kWalk;
+      } else {
+        k += G;
+      }
+      return mine;
+    }
+    return false;
+  }
+  __device__ __forceinline__ void result(MarchResult& res) const {
+    res.T = T;
+    res.n_samples = nsamp;
+    res.depth = depth;
+    res.n_bricks = nbr;
+  }
+};
+
 // Whether the lanes waiting for a tile step run it in this iteration: a wavefront of diverged lanes
 // issues every phase that any of its lanes is in, each iteration.  The tile step (tile walk, slab
 // test, twelve divisions) costs more vector instructions than the cell and sample steps together
@@ -545,53 +733,6 @@ __device__ __forceinline__ void view_encoding(V3 d, float e[15]) {
   }
 }
 
-// ---------------------------------------------------------------------------- per-lane FP32 MLP
-// Activations live in a lane-private LDS column (entry k of lane t at xs[k * 64], wavefront-sized
-// blocks), weights in the f32t layout Wt[in][out4] then b[out4].
-// One dense layer for one lane: y = b + x Wt, x read from this lane's LDS column (stride 64),
-// Wt rows read as float4 (all lanes of a wave in one tile read the same address).
-template <int IN, int OUT>
-__device__ __forceinline__ void dense_f32(const float* __restrict__ Wt, const float* __restrict__ b,
-                                          const float* xs, float (&y)[OUT]) {
-  static_assert(OUT % 4 == 0, "padded width");
-#pragma unroll
-  for (int j = 0; j < OUT; ++j) y[j] = b[j];
-#pragma unroll 1
-  for (int i = 0; i < IN; ++i) {
-    const float xi = xs[i * 64];
-    const float4* w = reinterpret_cast<const float4*>(Wt + i * OUT);
-#pragma unroll
-    for (int j = 0; j < OUT / 4; ++j) {
-      const float4 q = w[j];
-      y[4 * j + 0] = __builtin_fmaf(xi, q.x, y[4 * j + 0]);
-      y[4 * j + 1] = __builtin_fmaf(xi, q.y, y[4 * j + 1]);
-      y[4 * j + 2] = __builtin_fmaf(xi, q.z, y[4 * j + 2]);
-      y[4 * j + 3] = __builtin_fmaf(xi, q.w, y[4 * j + 3]);
-    }
-  }
-}
-
-// Per-sample MLP on one lane: input in xs[0..IN), hidden layers ReLU, sigmoid RGB.
-template <int IN, int WD, int L>
-__device__ __forceinline__ void mlp_f32(const float* __restrict__ P, float* xs, float rgb[3]) {
-  float y[WD];
-  dense_f32<IN, WD>(P, P + IN * WD, xs, y);
-  P += IN * WD + WD;
-#pragma unroll
-  for (int j = 0; j < WD; ++j) xs[j * 64] = y[j] > 0.0f ? y[j] : 0.0f;
-#pragma unroll 1
-  for (int l = 1; l < L - 1; ++l) {
-    dense_f32<WD, WD>(P, P + WD * WD, xs, y);
-    P += WD * WD + WD;
-#pragma unroll
-    for (int j = 0; j < WD; ++j) xs[j * 64] = y[j] > 0.0f ? y[j] : 0.0f;
-  }
-  float z[4];
-  dense_f32<WD, 4>(P, P + WD * 4, xs, z);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) rgb[c] = sigmoid_cw(z[c]);
-}
-
 template <bool HALF>
 struct FeatLoad;
 template <>
@@ -614,29 +755,6 @@ struct FeatLoad<false> {  // 4 floats per 16-byte load, raw bits ANDed with m
     v[2] = __uint_as_float(q.z & m); v[3] = __uint_as_float(q.w & m);
   }
 };
-
-// Trilinear features of one sample into this lane's LDS column xs[0..F).
-template <int F, bool HALF>
-__device__ __forceinline__ void gather_features(const void* __restrict__ feats, const Corners& c, float* xs) {
-  using LD = FeatLoad<HALF>;
-  constexpr int V = LD::kVec;
-  static_assert(F % V == 0, "feature dim must fill whole 16-byte vectors");
-  uint32_t m[8];  // computed ahead of the loads: the masking statements bound scheduling regions
-#pragma unroll
-  for (int k = 0; k < 8; ++k) m[k] = corner_mask(c.slot[k] >= 0);
-#pragma unroll
-  for (int ch = 0; ch < F / V; ++ch) {
-    float v[8][V];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)  // unconditional loads (slot 0 for empty corners), masked to zero
-      LD::load(feats, (int64_t)(c.slot[k] >= 0 ? c.slot[k] : 0) * F + ch * V, m[k], v[k]);
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      const float q[8] = {v[0][e], v[1][e], v[2][e], v[3][e], v[4][e], v[5][e], v[6][e], v[7][e]};
-      xs[(ch * V + e) * 64] = tri_combine(q, c.wx, c.wy, c.wz);
-    }
-  }
-}
 
 // Ray index of lane `tid` of a launch over n rays.  With image_width W > 0 (and W % 8 == 0,
 // rows % 8 == 0) each 64-lane wavefront takes an 8x8 pixel packet, so its rays stay coherent.

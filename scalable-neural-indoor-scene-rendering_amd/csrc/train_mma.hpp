@@ -3,6 +3,7 @@
 #pragma once
 
 #include "mfma_ops.hpp"
+#include "snisr_device.hpp"
 
 namespace snisr {
 
@@ -166,6 +167,38 @@ __device__ __forceinline__ void mma_blocks(const float* __restrict__ A, const fl
 
 __device__ __forceinline__ void store4(float* p, const float* v) {
   *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// Trilinear features of one record into the row order of the products: x[s] = feature tr_row(s, h) for
+// the steps whose 8-row group holds features.  The loads are unconditional (empty corners read slot 0,
+// which exists, and mask[q] zeroes their raw bits), so a group's eight loads are in flight together.
+template <int F, bool HALF>
+__device__ __forceinline__ void gather_rows(const void* __restrict__ feats, const Corners& cn, const uint32_t (&mask)[8],
+                                            int h, float* x) {
+  static_assert(F % 8 == 0 && F <= 32, "feature rows must fill whole 8-row groups of the first block");
+#pragma unroll
+  for (int g = 0; g < F / 8; ++g) {
+    float v[8][4];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int64_t off = (int64_t)(cn.slot[q] >= 0 ? cn.slot[q] : 0) * F + 8 * g + 4 * h;
+      if (HALF) {
+        uint2 raw = *reinterpret_cast<const uint2*>(reinterpret_cast<const _Float16*>(feats) + off);
+        raw.x &= mask[q];
+        raw.y &= mask[q];
+        const _Float16* hv = reinterpret_cast<const _Float16*>(&raw);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[q][t] = (float)hv[t];
+      } else {
+        FeatLoad<false>::load(feats, off, mask[q], v[q]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float qv[8] = {v[0][t], v[1][t], v[2][t], v[3][t], v[4][t], v[5][t], v[6][t], v[7][t]};
+      x[4 * g + t] = tri_combine(qv, cn.wx, cn.wy, cn.wz);
+    }
+  }
 }
 
 }  // namespace snisr

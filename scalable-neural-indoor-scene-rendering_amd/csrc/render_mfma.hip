@@ -308,56 +308,64 @@ static int64_t render_layout(int64_t n, int64_t cpr, int64_t samples, int32_t T,
   return off;
 }
 
-// ------------------------------------------------------------------------- march passes
-template <int MODE>  // 0: count, 1: emit records, 2: emit records + training extras
-__global__ __launch_bounds__(64) void k_march_pass(snisr_scene S, snisr_march_params P, snisr_rays R,
-                                                   snisr_render_out O, Workspace W, int packet_w, int enc_dtype,
-                                                   const int32_t* __restrict__ order) {
-  const int64_t tid = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (tid >= R.n) return;
-  const int64_t i = order ? (int64_t)order[tid] : ray_of_thread(tid, R.n, packet_w);
-  const float* og = R.origins + i * R.origin_stride;
-  const V3 origin = v3(og[0], og[1], og[2]);
-  const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
-  const float t_hit = R.t_hit ? R.t_hit[i] : __builtin_inff();
-  const int32_t* vis = R.visited ? R.visited + i * P.max_tiles : nullptr;
-  MarchResult res;
-  if (MODE > 0) {
-    const int64_t base = W.offsets[i];
-    int64_t k = base;
-    bool over = false;
-    march_ray_any(packet_w > 0 && !order, S, P, origin, d, t_hit, vis, nullptr, 0,
-              [&](int tile, const V3& f, const Corners&, float w, float sig, float interval, float T_after) {
-                if (k < W.cap) {
-                  W.rec_f[k] = make_float4(f.x, f.y, f.z, w);
-                  W.rec_ti[k] = make_int2(tile, (int)i);
-                  if (MODE == 2) W.rec_b[k] = make_float4(interval, T_after, sig, 0.0f);
-                } else {
-                  over = true;
-                }
-                ++k;
-              },
-              res);
-    if (over) *W.overflow = 1;
-  } else {
-    int32_t* bricks = O.bricks ? O.bricks + i * O.brick_cap : nullptr;
-    march_ray_any(packet_w > 0 && !order, S, P, origin, d, t_hit, vis, bricks, O.brick_cap, [&](int, const V3&, const Corners&, float, float, float, float) {}, res);
-    if (bricks)
-      for (int k = res.n_bricks; k < O.brick_cap; ++k) bricks[k] = -1;
-    W.counts[i] = res.n_samples;
-    float enc[15];
-    view_encoding(d, enc);
-    uint16_t e16[16];
+// the 15-value view encoding of a unit direction in the MLP's operand type, 32 bytes per ray
+__device__ __forceinline__ void write_encoding(V3 d, int enc_dtype, uint16_t* out) {
+  float enc[15];
+  view_encoding(d, enc);
+  uint16_t e16[16];
 #pragma unroll
-    for (int k = 0; k < 15; ++k) e16[k] = to_bits(enc[k], enc_dtype);
-    e16[15] = 0;
-    uint4* dst = reinterpret_cast<uint4*>(W.enc + i * 16);
-    dst[0] = *reinterpret_cast<const uint4*>(e16);
-    dst[1] = *reinterpret_cast<const uint4*>(e16 + 8);
-    if (O.T) O.T[i] = res.T;
-    if (O.n_samples) O.n_samples[i] = res.n_samples;
-    if (O.depth) O.depth[i] = res.depth;
+  for (int k = 0; k < 15; ++k) e16[k] = to_bits(enc[k], enc_dtype);
+  e16[15] = 0;
+  uint4* dst = reinterpret_cast<uint4*>(out);
+  dst[0] = *reinterpret_cast<const uint4*>(e16);
+  dst[1] = *reinterpret_cast<const uint4*>(e16 + 8);
+}
+
+// ------------------------------------------------------------------------- march passes
+// A training march pass, every ray on a group of G lanes (march_group_lanes; with one ray per lane the two
+// passes took 172 us of the 332 us step of 3,001 rays in one tile, which takes 274 us now)
+template <bool EMIT, int G>  // count the samples, or write their records with the training extras
+__global__ __launch_bounds__(64) void k_march_pass(snisr_scene S, snisr_march_params P, snisr_rays R,
+                                                         snisr_render_out O, Workspace W, int enc_dtype) {
+  const int g = (int)threadIdx.x % G;
+  const int64_t i = (int64_t)blockIdx.x * (64 / G) + threadIdx.x / G;
+  if (i >= R.n) return;  // whole groups
+  const float* og = R.origins + i * R.origin_stride;
+  const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
+  int32_t* bricks = !EMIT && O.bricks ? O.bricks + i * O.brick_cap : nullptr;
+  GroupMarch<G> m;
+  m.init(S, P, v3(og[0], og[1], og[2]), d, R.t_hit ? R.t_hit[i] : __builtin_inff(),
+         R.visited ? R.visited + i * P.max_tiles : nullptr);
+  const int64_t base = EMIT ? W.offsets[i] : 0;
+  bool over = false;
+  while (m.phase != GroupMarch<G>::kDone) {
+    const bool turn = tile_quorum(m.phase == GroupMarch<G>::kTile);
+    m.step(S, P, turn, bricks, O.brick_cap,
+           [&](int tile, const V3& f, const Corners&, float w, float sig, float interval, float T_after, int idx) {
+             if (EMIT) {
+               const int64_t k = base + idx;
+               if (k < W.cap) {
+                 W.rec_f[k] = make_float4(f.x, f.y, f.z, w);
+                 W.rec_ti[k] = make_int2(tile, (int)i);
+                 W.rec_b[k] = make_float4(interval, T_after, sig, 0.0f);
+               } else {
+                 over = true;
+               }
+             }
+           });
   }
+  if (EMIT) {
+    if (over) *W.overflow = 1;
+    return;
+  }
+  if (g != 0) return;
+  if (bricks)
+    for (int k = m.nbr; k < O.brick_cap; ++k) bricks[k] = -1;
+  W.counts[i] = m.nsamp;
+  write_encoding(d, enc_dtype, W.enc + i * 16);
+  if (O.T) O.T[i] = m.T;
+  if (O.n_samples) O.n_samples[i] = m.nsamp;
+  if (O.depth) O.depth[i] = m.depth;
 }
 
 // ------------------------------------------------------------------------- exclusive scan
@@ -741,15 +749,7 @@ __global__ __launch_bounds__(64) void k_march_render(snisr_scene S, snisr_march_
     if (bricks)
       for (int b = res.n_bricks; b < O.brick_cap; ++b) bricks[b] = -1;
     W.counts[i] = res.n_samples;
-    float enc[15];
-    view_encoding(d, enc);
-    uint16_t e16[16];
-#pragma unroll
-    for (int q = 0; q < 15; ++q) e16[q] = to_bits(enc[q], enc_dtype);
-    e16[15] = 0;
-    uint4* dst = reinterpret_cast<uint4*>(W.enc + i * 16);
-    dst[0] = *reinterpret_cast<const uint4*>(e16);
-    dst[1] = *reinterpret_cast<const uint4*>(e16 + 8);
+    write_encoding(d, enc_dtype, W.enc + i * 16);
     if (O.T) O.T[i] = res.T;
     if (O.n_samples) O.n_samples[i] = res.n_samples;
     if (O.depth) O.depth[i] = res.depth;
@@ -769,22 +769,14 @@ __global__ __launch_bounds__(256) void k_ray_enc(snisr_rays R, RenderWs W, int e
   const int64_t i = r0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= r1) return;
   const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
-  float enc[15];
-  view_encoding(d, enc);
-  uint16_t e16[16];
-#pragma unroll
-  for (int q = 0; q < 15; ++q) e16[q] = to_bits(enc[q], enc_dtype);
-  e16[15] = 0;
-  uint4* dst = reinterpret_cast<uint4*>(W.enc + i * 16);
-  dst[0] = *reinterpret_cast<const uint4*>(e16);
-  dst[1] = *reinterpret_cast<const uint4*>(e16 + 8);
+  write_encoding(d, enc_dtype, W.enc + i * 16);
 }
 
 // The march of arbitrary rays (no pixel packets, or a ray schedule) as a queue: a wavefront's lanes
 // take rays (thread indices tid0 .. tid1 - 1, ray = order[tid] or tid) from a per-chunk counter and,
 // when a quarter of the lanes have finished theirs, take new ones together, so that a wavefront is
 // not held by its longest ray while most lanes idle.  Each ray is marched exactly as by
-// march_ray_flat (same steps, same records), only the lanes that run it change.  The grid is sized
+// march_ray (FlatMarch: same steps, same records), only the lanes that run it change.  The grid is sized
 // to the device's resident wavefronts; every wavefront ends once the counter passes tid1 and its
 // lanes' rays are done.
 constexpr int kRefillQuorum = 4;
@@ -879,6 +871,69 @@ __global__ __launch_bounds__(64) void k_march_queue(snisr_scene S, snisr_march_p
     if (wsum) atomicAdd((unsigned long long*)W.total, (unsigned long long)wsum);
     if (wmx) atomicMax(W.max_count, wmx);
     if (wmx > W.cpr) *W.overflow = 1;
+  }
+}
+
+// The march of a batch or frame too small to fill the device with one ray per lane (march_group_lanes):
+// rays in groups of G lanes (GroupMarch), 64 / G rays per wavefront, each sample's record written by the lane that took it (a group's eight records are one 128-byte line).
+template <int G>
+__global__ __launch_bounds__(64) void k_march_group(snisr_scene S, snisr_march_params P, snisr_rays R,
+                                                    snisr_render_out O, RenderWs W, int packet_w, int enc_dtype,
+                                                    const int32_t* __restrict__ order, int64_t tid0, int64_t tid1) {
+  const int lane = threadIdx.x, g = lane % G;
+  const int64_t tid = tid0 + (int64_t)blockIdx.x * (64 / G) + lane / G;
+  int ns = 0;
+  if (tid < tid1) {  // whole groups
+    const int64_t i = order ? (int64_t)order[tid] : ray_of_thread(tid, R.n, packet_w);
+    const float* og = R.origins + i * R.origin_stride;
+    const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
+    const int cpr = W.cpr;
+    const int64_t slot0 = i * (int64_t)cpr;
+    int32_t* bricks = O.bricks ? O.bricks + i * O.brick_cap : nullptr;
+    GroupMarch<G> m;
+    m.init(S, P, v3(og[0], og[1], og[2]), d, R.t_hit ? R.t_hit[i] : __builtin_inff(),
+           R.visited ? R.visited + i * P.max_tiles : nullptr);
+    int run_tile = -1, run_start = 0;
+    RunList rl;
+    rl.reset();
+    // every lane of the group keeps the runs; the first one stores those past the registers
+    auto close_run = [&](int end) {
+      const int v = run_tile | ((end - run_start) << 16);
+      if (g == 0 || rl.n < 4) rl.add(v, W.rec_t + slot0);
+      else ++rl.n;
+    };
+    while (m.phase != GroupMarch<G>::kDone) {
+      const bool turn = tile_quorum(m.phase == GroupMarch<G>::kTile);
+      const int before = m.nsamp;
+      m.step(S, P, turn, bricks, O.brick_cap,
+             [&](int, const V3& f, const Corners&, float w, float, float, float, int idx) {
+               if (idx < cpr) W.rec_f[slot0 + idx] = make_float4(f.x, f.y, f.z, w);
+             });
+      if (m.nsamp > before && before < cpr && m.tile != run_tile) {
+        if (run_tile >= 0) close_run(before);
+        run_tile = m.tile;
+        run_start = before;
+      }
+    }
+    if (run_tile >= 0) close_run(min(m.nsamp, cpr));
+    if (g == 0) {
+      rl.store(W.runs4 + i);
+      if (bricks)
+        for (int b = m.nbr; b < O.brick_cap; ++b) bricks[b] = -1;
+      W.counts[i] = m.nsamp;
+      write_encoding(d, enc_dtype, W.enc + i * 16);
+      if (O.T) O.T[i] = m.T;
+      if (O.n_samples) O.n_samples[i] = m.nsamp;
+      if (O.depth) O.depth[i] = m.depth;
+      ns = m.nsamp;
+    }
+  }
+  const int64_t sum = wave_sum_i64((int64_t)ns);
+  const int mx = wave_max_i32(ns);
+  if (lane == 0) {
+    if (sum) atomicAdd((unsigned long long*)W.total, (unsigned long long)sum);
+    if (mx) atomicMax(W.max_count, mx);
+    if (mx > W.cpr) *W.overflow = 1;
   }
 }
 
@@ -1677,6 +1732,25 @@ int device_cus() {
   return v;
 }
 
+// Lanes per ray of a march over n rays (GroupMarch); 1: one ray per lane (the packet or queue march).
+// A group finds its ray's cells and samples in fewer dependent memory round trips but repeats the
+// walk's arithmetic on each of its lanes, so it pays while the launch has too few wavefronts to cover
+// the waits.  Measured on 256 CUs, whole render in us (27-tile batch | single-tile view | 16-tile room):
+//   n = 5-6k     one lane 386 | 297 | 620     8 lanes 153 | 59 | 113       4 lanes 176 | 68 | 128
+//   n = 20k      one lane 428                 8 lanes 233                  4 lanes 228      2 lanes 287
+//   n = 50-56k   one lane 530 | 258 | 465     4 lanes 384 | 84 | 256       2 lanes 369 | 95 | 253
+//   n = 127k     one lane       233 | 533     4 lanes       124 | 446      2 lanes       115 | 383
+//   n = 200-230k one lane 1087 | 230 | 695    2 lanes 1032 | 146 | 607
+//   n = 400k     one lane 1999                2 lanes 1999
+//   n = 515k     one lane       270 | 1130    2 lanes       236 | 1212
+// Training (no queue march behind it) keeps two lanes at every larger size: 128k rays 4404 -> 4213.
+static int march_group_lanes(int64_t n, bool packets) {
+  const int64_t cus = device_cus();
+  if (n <= 64 * cus) return 8;
+  if (n <= 224 * cus) return 4;
+  return n <= (packets ? 1024 : 1536) * cus ? 2 : 1;
+}
+
 // resident wavefronts per CU of the queue-fed march (its grid covers the device once), per device
 static int march_queue_waves_per_cu() {
   static std::atomic<int> per[64];
@@ -1813,6 +1887,20 @@ int snisr_render_mfma_tuned(const snisr_scene* scene, const snisr_march_params* 
   // the shaded half of the render on one chunk's view: tile sort, MFMA MLP, per-ray reduction
   auto launch_march = [&](int64_t r0, int64_t r1, const int32_t* order, int c) -> int {
     const int64_t units = (r1 - r0 + 63) / 64;
+    const int lanes = march_group_lanes(r1 - r0, pw > 0 && !order);
+    if (lanes > 1) {
+      const dim3 ggrid((unsigned)(((r1 - r0) * lanes + 63) / 64));
+#define SNISR_MARCH_GROUP(G_)                                                                              \
+      if (lanes == G_)                                                                                     \
+        hipLaunchKernelGGL(k_march_group<G_>, ggrid, dim3(64), 0, st, *scene, *params, *rays, *out, W,     \
+                           order ? 0 : pw, dt, order, r0, r1);
+      SNISR_MARCH_GROUP(8)
+      SNISR_MARCH_GROUP(4)
+      SNISR_MARCH_GROUP(2)
+#undef SNISR_MARCH_GROUP
+      SNISR_LAUNCHED();
+      return SNISR_OK;
+    }
     if (pw > 0 && !order) {
       hipLaunchKernelGGL(k_march_render, dim3((unsigned)units), dim3(64), 0, st, *scene, *params, *rays, *out,
                          W, pw, dt, order, r0, r1);
@@ -1987,8 +2075,6 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   const int F = scene->feat_dim, WD = scene->mlp_width, L = scene->mlp_layers;
   const bool half = scene->feat_dtype == SNISR_F16;
   hipStream_t st = (hipStream_t)stream;
-  const int pw = packet_width(*rays);
-  const dim3 mgrid((unsigned)((n + 63) / 64));
   const int64_t nblocks = (n + kScanTile - 1) / kScanTile;
   bool ok = false;
 #define SNISR_CHECK_SHAPE(F_, W_, L_, H_) ok = ok || (F == F_ && WD == W_ && L == L_ && half == H_);
@@ -1997,9 +2083,14 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   SNISR_REQUIRE(ok, SNISR_ERR_SHAPE, "train_forward: unsupported shape F=%d width=%d layers=%d", F, WD, L);
   SNISR_HIP(stage_event(out, 0, st));
   // no ray schedule: sorting arbitrary training rays by (first tile, octant) made the march slower
-  const int32_t* order = nullptr;
-  hipLaunchKernelGGL(k_march_pass<0>, mgrid, dim3(64), 0, st, *scene, *params, *rays, *out, W, pw, (int)SNISR_F16,
-                     order);
+  const int lanes = march_group_lanes(n, false) > 2 ? march_group_lanes(n, false) : 2;
+  const dim3 mgrid((unsigned)((n * lanes + 63) / 64));
+#define SNISR_MARCH_PASS(EMIT_, G_)                                                                                   \
+  if (lanes == G_)                                                                                                    \
+    hipLaunchKernelGGL((k_march_pass<EMIT_, G_>), mgrid, dim3(64), 0, st, *scene, *params, *rays, *out, W, (int)SNISR_F16);
+  SNISR_MARCH_PASS(false, 8)
+  SNISR_MARCH_PASS(false, 4)
+  SNISR_MARCH_PASS(false, 2)
   SNISR_LAUNCHED();
   hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nblocks), dim3(kScanBlock), 0, st, W.counts, n, W.offsets,
                      W.block_sums);
@@ -2009,8 +2100,10 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   SNISR_LAUNCHED();
   hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nblocks), dim3(kScanBlock), 0, st, W.offsets, n, W.block_sums);
   SNISR_LAUNCHED();
-  hipLaunchKernelGGL(k_march_pass<2>, mgrid, dim3(64), 0, st, *scene, *params, *rays, *out, W, pw, (int)SNISR_F16,
-                     order);
+  SNISR_MARCH_PASS(true, 8)
+  SNISR_MARCH_PASS(true, 4)
+  SNISR_MARCH_PASS(true, 2)
+#undef SNISR_MARCH_PASS
   SNISR_LAUNCHED();
   hipLaunchKernelGGL(k_tile_hist, dim3(kSortGrid), dim3(kSortBlock), 0, st, W);
   SNISR_LAUNCHED();

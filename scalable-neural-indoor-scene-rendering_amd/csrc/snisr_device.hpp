@@ -402,7 +402,7 @@ struct FlatMarch {
     far_ = fminx(fminx(tmax[0], tmax[1]), tmax[2]);
   }
   // One unit of work.  A lane waiting for a tile step does nothing unless `tile_turn` (see
-  // march_ray_flat).
+  // tile_quorum).
   template <class OnSample>
   __device__ __forceinline__ void step(const snisr_scene& S, const snisr_march_params& P, bool tile_turn,
                                        int32_t* bricks, int brick_cap, OnSample&& on_sample) {
@@ -689,33 +689,6 @@ __device__ __forceinline__ bool tile_quorum(bool waiting) {
   const uint64_t live = __builtin_amdgcn_ballot_w64(true);
   const uint64_t wait = __builtin_amdgcn_ballot_w64(waiting);
   return wait == live || kTileQuorum * __builtin_popcountll(wait) >= __builtin_popcountll(live);
-}
-
-template <class OnSample>
-__device__ __forceinline__ void march_ray_flat(const snisr_scene& S, const snisr_march_params& P, V3 origin, V3 d,
-                                               float t_hit, const int32_t* __restrict__ vis, int32_t* bricks,
-                                               int brick_cap, OnSample&& on_sample, MarchResult& res) {
-  FlatMarch m;
-  m.init(S, P, origin, d, t_hit, vis);
-  // the ballots at the head of the single loop also keep the compiler from turning the phase
-  // machine back into nested loops
-  while (m.phase != FlatMarch::kDone) {
-    const bool turn = tile_quorum(m.phase == FlatMarch::kTile);
-    m.step(S, P, turn, bricks, brick_cap, on_sample);
-  }
-  m.result(res);
-}
-
-// Camera packets (8x8 pixels per wavefront) walk nearly the same cells in the same order, so the
-// nested loops of march_ray keep their lanes together; arbitrary rays (training batches, batched
-// tiles) diverge, and the flattened loop is faster for them (measured 2.5-2.8x on such batches,
-// 0.55x on camera packets).
-template <class OnSample>
-__device__ __forceinline__ void march_ray_any(bool packets, const snisr_scene& S, const snisr_march_params& P,
-                                              V3 origin, V3 d, float t_hit, const int32_t* __restrict__ vis,
-                                              int32_t* bricks, int brick_cap, OnSample&& on_sample, MarchResult& res) {
-  if (packets) march_ray(S, P, origin, d, t_hit, vis, bricks, brick_cap, on_sample, res);
-  else march_ray_flat(S, P, origin, d, t_hit, vis, bricks, brick_cap, on_sample, res);
 }
 
 // 15-d view encoding Positional_Encoding(L=2) (training/scripts/networks.py:8-13) of a unit dir.

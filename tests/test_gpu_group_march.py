@@ -42,3 +42,39 @@ def test_fp32_render_matches_oracle(oracle_mod, width, n):
         for k in ("T", "depth"):
             assert np.array_equal(g[k].view(np.uint32), ref[k].view(np.uint32)), k
         assert np.abs(g["rgb"] - ref["rgb"]).max() <= RGB_TOL
+
+
+# batches on either side of the group sizes: 8 lanes per ray up to 64 rays per CU, 4 up to 224, then 2
+@pytest.mark.parametrize("n", [1, 9, 64, 16384, 16391, 57344, 57351])
+def test_small_batches_match_fp32_path(n):
+    from snisr import _native as N
+    from snisr import train as TRN
+    sc = scene(64)
+    ds = D.DeviceScene(sc, mfma_dtype=N.SNISR_F16)
+    o, d, th = rays(n, n)
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    for hit in (None, t(th)):
+        ref = D.render_fp32(ds, t(o), t(d), t_hit=hit, brick_cap=24)
+        out = D.render_mfma(ds, t(o), t(d), t_hit=hit, brick_cap=24)
+        for k in ("n_samples", "T", "depth", "bricks"):
+            assert torch.equal(out[k].view(torch.int32), ref[k].view(torch.int32)), k
+        assert (out["rgb"] - ref["rgb"]).abs().max() <= 5e-3   # FP16 layers
+        trn, _ = TRN.train_forward(ds, t(o), t(d), t_hit=hit)
+        for k in ("n_samples", "T", "depth"):
+            assert torch.equal(trn[k].view(torch.int32), ref[k].view(torch.int32)), k
+        assert (trn["rgb"] - ref["rgb"]).abs().max() <= 2e-5
+
+
+@pytest.mark.parametrize("H,W", [(8, 8), (64, 96), (60, 96), (248, 232)])
+def test_small_frames_match_fp32_path(H, W):
+    from snisr import _native as N
+    sc = scene(64)
+    ds = D.DeviceScene(sc, mfma_dtype=N.SNISR_F16)
+    cam = S.room_camera(3, (0, 0, 0), (3, 2, 2), H, W, focal=0.6 * W)
+    d = torch.from_numpy(S.camera_rays_np(cam)).to(DEV)
+    o = torch.from_numpy(cam.origin).to(DEV)
+    ref = D.render_fp32(ds, o, d, image_width=W)
+    out = D.render_mfma(ds, o, d, image_width=W)
+    for k in ("n_samples", "T", "depth"):
+        assert torch.equal(out[k].view(torch.int32), ref[k].view(torch.int32)), k
+    assert (out["rgb"] - ref["rgb"]).abs().max() <= 5e-3

@@ -7,13 +7,13 @@
 // outputs, LeakyReLU 0.01) of the reference's training configuration (training/config/cfg.yaml:38-46),
 // used for the compute_voxels bake, the background samples and the specular branch.
 //
-// FP32 MFMA (v_mfma_f32_32x32x2_f32) with the training chain's fragment layout: a wavefront takes 32
-// samples as the 32 columns, computes their positional encoding cooperatively (30 sin/cos pairs per
-// sample spread over the lanes, through LDS), and every layer's output (the D layout) is the next
-// layer's B operand, so activations never leave registers.  The weights are packed once per call as
-// forward and transposed fragments.  The forward writes only the outputs.  The backward recomputes
-// the forward from the points, keeps the activation signs as bit masks, writes each layer's input
-// row and output-delta row, and reduces the weight gradients dW = sum delta (x) input on FP32 MFMA.
+// The products run on FP16 MFMA with every FP32 operand as two parts (train_mma.hpp): a wavefront takes 32
+// samples as the 32 columns, each half of a sample's two lanes computes half of its positional encoding
+// (15 sin/cos pairs), and every layer's output (the D layout) is the next layer's B operand, so activations never leave registers; the four wavefronts of a workgroup share
+// the weights, packed once per call as forward and transposed fragments, through LDS.  The forward writes
+// only the outputs.  The backward recomputes the forward from the points, keeps the activation signs as bit
+// masks, writes each layer's input row and output-delta row, and a second kernel reduces the weight
+// gradients dW = sum delta (x) input from the rows.
 #include "snisr_common.hpp"
 #include "snisr_device.hpp"
 #include "train_dw.hpp"
@@ -55,10 +55,55 @@ __host__ __device__ inline int64_t pe_d_off(int l, int L, int depth, int n_out, 
 }
 
 constexpr int kPIn = 63;                 // encoding width (3 + 6 L)
-constexpr int kPNs0 = tr_ns0(kPIn);      // input steps of layer 0 (rows 0..63, row 63 zero)
-constexpr int kPeLds = 65;               // LDS row pitch of the encoding (conflict-free column reads)
+constexpr int kPNs0 = tr_ns0(kPIn);      // input registers of layer 0 (rows 0..63)
 
-// float offsets of the packed fragments (one block of tr_stride(63, 64, depth, n_out) floats)
+// The encoding's inputs in layer 0's row order: lane half h holds the bands 5h .. 5h+4, so that no value
+// crosses lanes.  Register s of half h: s = 0: x or z; s = 1: y or nothing; then band by band sin x, sin y,
+// sin z, cos x, cos y, cos z.  pe_input(row) is the input at a row (63: none), row = tr_row(s, h).
+__host__ __device__ constexpr int pe_input(int row) {
+  const int h = (row / 4) % 2, s = 16 * (row / 32) + 4 * (row % 32 / 8) + row % 4;
+  if (s < 2) return h == 0 ? s : (s == 0 ? 2 : 63);
+  return 3 + 30 * h + s - 2;
+}
+
+// sin and cos of 2^f v for f = 5h .. 5h+4, h = lane half.  v / (2 pi) is formed once as hi + lo; scaling it by
+// 2^f is exact, and so is taking off the nearest quarter turn, so every band starts from an angle within
+// pi / 4 that carries the rounding of that quotient's 48 bits only; Taylor's series to the 9th and 10th
+// power are then below half an ulp.  Above 2^12 (a band then passes 2^21 turns) the library function takes
+// over for the whole wavefront.
+__device__ __forceinline__ void pe_bands(float v, int h, float (&sn)[5], float (&cs)[5]) {
+  constexpr float k1 = 0.15915494309189535f;                        // 1 / (2 pi) rounded
+  constexpr float k2 = (float)(0.15915494309189533577 - (double)k1);
+  constexpr float turn = 6.283185307179586f;
+  float f = h ? 32.0f : 1.0f;
+  if (__builtin_amdgcn_ballot_w64(!(fabsf(v) < 4096.0f))) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q, f *= 2.0f) sincosf(f * v, &sn[q], &cs[q]);
+    return;
+  }
+  const float hi = v * k1, lo = __builtin_fmaf(v, k2, __builtin_fmaf(v, k1, -hi));
+#pragma unroll
+  for (int q = 0; q < 5; ++q, f *= 2.0f) {
+    const float a = f * hi, n = __builtin_rintf(4.0f * a);
+    const float u = __builtin_fmaf(f, lo, __builtin_fmaf(-0.25f, n, a)) * turn, u2 = u * u;
+    float s = 2.7557319e-6f, c = -2.7557319e-7f;
+    s = __builtin_fmaf(s, u2, -1.9841270e-4f);
+    s = __builtin_fmaf(s, u2, 8.3333333e-3f);
+    s = __builtin_fmaf(s, u2, -1.6666667e-1f);
+    s = __builtin_fmaf(s * u2, u, u);
+    c = __builtin_fmaf(c, u2, 2.4801587e-5f);
+    c = __builtin_fmaf(c, u2, -1.3888889e-3f);
+    c = __builtin_fmaf(c, u2, 4.1666667e-2f);
+    c = __builtin_fmaf(c, u2, -0.5f);
+    c = __builtin_fmaf(c, u2, 1.0f);
+    const int quad = (int)n;
+    const float x = quad & 1 ? c : s, y = quad & 1 ? s : c;
+    sn[q] = quad & 2 ? -x : x;
+    cs[q] = (quad + 1) & 2 ? -y : y;
+  }
+}
+
+// floats of the packed fragments
 __host__ __device__ inline int64_t pe_frag_floats(int depth, int n_out) { return tr_stride(kPIn, kPW, depth, n_out); }
 
 __device__ __forceinline__ float leaky_mask(uint64_t m, int r, float v, float slope) {
@@ -66,103 +111,88 @@ __device__ __forceinline__ float leaky_mask(uint64_t m, int r, float v, float sl
 }
 
 // One wavefront = 32 samples.  Forward (BWD false): out[j][0..NOUT).  Backward: recomputes the
-// forward, stores each layer's input row (pitch 64) and output-delta row (pitch 64, the last layer
-// NOUT) for the weight-gradient reduction.
+// forward, stores each layer's input rows (pitch 64) and output-delta rows (pitch 64, the last layer
+// NOP) for the weight-gradient reduction.  chunks: weight chunks the kernel reads; bias: float offset of the
+// biases in P.
 template <int NOUT, bool BWD>
-__global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ P, const float* __restrict__ pts,
-                                                      int64_t n, int depth, float slope, float* __restrict__ out,
-                                                      const float* __restrict__ g_out, float* __restrict__ rows) {
+__global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ P, int chunks, int64_t bias_off,
+                                                      const float* __restrict__ pts, int64_t n, int depth, float slope,
+                                                      float* __restrict__ out, const float* __restrict__ g_out,
+                                                      float* __restrict__ rows) {
   static_assert(NOUT % 4 == 0 && NOUT <= 32, "output rows in whole 4-row groups of one block");
-  constexpr int NSBO = NOUT <= 8 ? 4 : 16;  // backward steps of the output layer
-  __shared__ float pe_lds[4 * 32 * kPeLds];
+  constexpr int NKO = (NOUT + 15) / 16;   // k-chunks of the output layer's transposed product
+  constexpr int NOP = NOUT <= 4 ? 4 : 32;  // delta pitch of the output layer
+  __shared__ __align__(16) uint8_t w_lds[2 * kChunkBytes];
   const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int64_t j0 = ((int64_t)blockIdx.x * 4 + wv) * 32;
-  if (j0 >= n) return;  // whole wavefront past the end (only wavefront-level LDS sharing below)
+  const bool any = j0 < n;  // else a wavefront past the end: it keeps the others' barriers
   const int64_t j = j0 + col;
   const bool valid = j < n;
-  float* E = pe_lds + wv * 32 * kPeLds;
-  // ---- positional encoding of the wavefront's 32 samples: [x, sin(2^f x), cos(2^f x)] (f < 10)
-  for (int q = lane; q < 32 * 30; q += 64) {
-    const int smp = q / 30, t = q - 30 * smp, f = t / 3, c = t - 3 * f;
-    const float v = j0 + smp < n ? pts[3 * (j0 + smp) + c] : 0.0f;
-    float sn, cs;
-    sincosf((float)(1 << f) * v, &sn, &cs);
-    E[smp * kPeLds + 3 + 6 * f + c] = sn;
-    E[smp * kPeLds + 6 + 6 * f + c] = cs;
-  }
-  for (int q = lane; q < 32 * 4; q += 64) {
-    const int smp = q >> 2, c = q & 3;
-    E[smp * kPeLds + (c < 3 ? c : kPIn)] = (c < 3 && j0 + smp < n) ? pts[3 * (j0 + smp) + c] : 0.0f;
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  FragStream fs;
+  fs.start(P, w_lds, chunks);
+  // ---- layer-0 inputs
   float x0[kPNs0];
+  {
+    float v[3];
 #pragma unroll
-  for (int s = 0; s < kPNs0; ++s) x0[s] = E[col * kPeLds + tr_row(s, h)];
-  // rows in the lane layout of the weight-gradient reduction (32-sample blocks, one 1 KB store per
-  // feature group and wavefront); the regions hold whole blocks
+    for (int c = 0; c < 3; ++c) v[c] = valid ? pts[3 * j + c] : 0.0f;
+    x0[0] = h ? v[2] : v[0];
+    x0[1] = h ? 0.0f : v[1];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      float sn[5], cs[5];
+      pe_bands(v[c], h, sn, cs);
+#pragma unroll
+      for (int q = 0; q < 5; ++q) {
+        x0[2 + 6 * q + c] = sn[q];
+        x0[5 + 6 * q + c] = cs[q];
+      }
+    }
+  }
   const int64_t in_rows = pe_rows(n) * kPW;  // floats of one layer's input rows
   const int64_t blk = j0;                    // first sample of this wavefront's block
-  if (BWD && valid) {
-#pragma unroll
-    for (int g = 0; g < kPNs0 / 4; ++g) store4(rows + blk * kPW + 256 * g + 4 * lane, x0 + 4 * g);
-  }
+  if (BWD && any) store_rows<kPW, kPNs0 / 4>(rows + blk * kPW, x0, lane);
   // ---- forward
+  const float* bias = P + bias_off;
   float a[32];
   uint64_t mask[8];
-  mma_blocks<kPNs0, 2>(
-      P + tr_fwd_off(kPIn, kPW, depth, 0), x0, lane,
-      [&](int ob) { return bias_block(P + tr_bias_off(kPIn, kPW, depth, 0), ob, h); },
-      [&](int ob, const f32x16& acc) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) a[ob * 16 + r] = acc[r] > 0.0f ? acc[r] : slope * acc[r];
-      });
+  const float* winv = P + bias_off + 64 * (depth - 1) + 32;
+  stream_layer<kPNs0 / 8, 2>(fs, x0, lane, winv[0], bias, [&](int r, float v) { a[r] = v > 0.0f ? v : slope * v; });
   uint64_t mk_last = 0;  // mask of the output layer's input
 #pragma unroll
   for (int l = 1; l < 8; ++l) {
+    bias += 64;
     mask[l] = 0;
 #pragma unroll
     for (int r = 0; r < 32; ++r) mask[l] |= (uint64_t)(a[r] > 0.0f) << r;
-    if (BWD && valid) {
-      float* Al = rows + l * in_rows + blk * kPW + 4 * lane;
-#pragma unroll
-      for (int g = 0; g < 8; ++g) store4(Al + 256 * g, a + 4 * g);
-    }
+    if (BWD && any) store_rows<kPW, 8>(rows + l * in_rows + blk * kPW, a, lane);
     if (l == depth - 1) {
       mk_last = mask[l];
       break;
     }
-    float b[32];
-    mma_blocks<32, 2>(
-        P + tr_fwd_off(kPIn, kPW, depth, l), a, lane,
-        [&](int ob) { return bias_block(P + tr_bias_off(kPIn, kPW, depth, l), ob, h); },
-        [&](int ob, const f32x16& acc) {
+    float y[32];
+    stream_layer<4, 2>(fs, a, lane, winv[l], bias, [&](int r, float v) { y[r] = v > 0.0f ? v : slope * v; });
 #pragma unroll
-          for (int r = 0; r < 16; ++r) b[ob * 16 + r] = acc[r] > 0.0f ? acc[r] : slope * acc[r];
-        });
-#pragma unroll
-    for (int r = 0; r < 32; ++r) a[r] = b[r];
+    for (int r = 0; r < 32; ++r) a[r] = y[r];
   }
-  // ---- output layer: rows 8 (r / 4) + 4 h + r % 4 of column col
-  if (!BWD) {
-    f32x16 z = bias_block(P + tr_bias_off(kPIn, kPW, depth, depth - 1), 0, h);
-    z = mma_f32_chain<32>(P + tr_fwd_off(kPIn, kPW, depth, depth - 1), a, z, lane);
+  // ---- output layer: rows 8 (r / 4) + 4 h + r % 4 of column col (the backward only steps over its weights)
+  if (BWD) {
+    fs.step();
+  } else {
+    float z[16];
+    stream_layer<4, 1>(fs, a, lane, winv[depth - 1], bias, [&](int r, float v) { z[r] = v; });
     if (valid) {
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        if (8 * g + 4 * h < NOUT) {
-          const float v[4] = {z[4 * g], z[4 * g + 1], z[4 * g + 2], z[4 * g + 3]};
-          store4(out + j * NOUT + 8 * g + 4 * h, v);
-        }
+        if (8 * g + 4 * h < NOUT) store4(out + j * NOUT + 8 * g + 4 * h, z + 4 * g);
     }
     return;
   }
-  // ---- backward: output delta (rows tr_row(s, h), s < NSBO), then d_{l-1} = (W_l^T d_l) * leaky'
+  // ---- backward: output delta (register s: row tr_row(s, h)), then d_{l-1} = (W_l^T d_l) * leaky'
   const int64_t d_base = (int64_t)depth * in_rows;  // delta rows follow the input rows
-  float dout[NSBO];
+  float dout[8 * NKO];
 #pragma unroll
-  for (int g = 0; g < NSBO / 4; ++g) {
+  for (int g = 0; g < 2 * NKO; ++g) {
     float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (valid && 8 * g + 4 * h < NOUT) v = *reinterpret_cast<const float4*>(g_out + j * NOUT + 8 * g + 4 * h);
     dout[4 * g] = v.x;
@@ -170,66 +200,52 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
     dout[4 * g + 2] = v.z;
     dout[4 * g + 3] = v.w;
   }
-  if (valid) {
-    constexpr int NOP = NOUT <= 4 ? 4 : 32;  // delta pitch of the output layer
-    float* Dl = rows + d_base + (int64_t)(depth - 1) * in_rows + blk * NOP;
-#pragma unroll
-    for (int g = 0; g < NSBO / 4; ++g)  // rows NOUT .. NOP - 1 carry zero deltas
-      if (8 * g + 4 * h < NOP) store4(Dl + lane_off(col, 8 * g + 4 * h), dout + 4 * g);
-  }
+  if (any) store_rows<NOP, NOP <= 4 ? 1 : 4>(rows + d_base + (int64_t)(depth - 1) * in_rows + blk * NOP, dout, lane);
   float d[32];
-  mma_blocks<NSBO, 2>(
-      P + tr_bwd_off(kPIn, kPW, depth, depth - 1, NOUT), dout, lane, [&](int) { return f32x16{}; },
-      [&](int ib, const f32x16& acc) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) d[ib * 16 + r] = leaky_mask(mk_last, ib * 16 + r, acc[r], slope);
-      });
+  stream_layer<NKO, 2>(fs, dout, lane, winv[depth - 1], nullptr,
+                       [&](int r, float v) { d[r] = leaky_mask(mk_last, r, v, slope); });
 #pragma unroll
   for (int l = 6; l >= 0; --l) {
     if (l > depth - 2) continue;
-    if (valid) {  // d = delta of layer l's outputs
-      float* Dl = rows + d_base + (int64_t)l * in_rows + blk * kPW + 4 * lane;
-#pragma unroll
-      for (int g = 0; g < 8; ++g) store4(Dl + 256 * g, d + 4 * g);
-    }
+    // d = delta of layer l's outputs
+    if (any) store_rows<kPW, 8>(rows + d_base + (int64_t)l * in_rows + blk * kPW, d, lane);
     if (l == 0) break;
     float e[32];
-    mma_blocks<32, 2>(
-        P + tr_bwd_off(kPIn, kPW, depth, l, NOUT), d, lane, [&](int) { return f32x16{}; },
-        [&](int ib, const f32x16& acc) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) e[ib * 16 + r] = leaky_mask(mask[l], ib * 16 + r, acc[r], slope);
-        });
+    stream_layer<4, 2>(fs, d, lane, winv[l], nullptr, [&](int r, float v) { e[r] = leaky_mask(mask[l], r, v, slope); });
 #pragma unroll
     for (int r = 0; r < 32; ++r) d[r] = e[r];
   }
 }
 
-// dW and db of layer blockIdx.y over split blockIdx.x of the samples (atomics into g_params)
-template <int IP, int OP, int INL, int OUTL>
+__global__ __launch_bounds__(kPackThreads) void k_pack_pe(const float* __restrict__ params, float* __restrict__ dst,
+                                                          int depth, int n_out) {
+  pack_train_layer(params, dst, kPIn, kPW, depth, blockIdx.x, n_out, [](int row) { return pe_input(row); });
+}
+
+// dW and db of layer blockIdx.y over split blockIdx.x of the 32-sample blocks (atomics into g_params)
+template <int IP, int OP, int INL, int OUTL, class InOf>
 __device__ void pe_dw_layer(const float* rows, int64_t n, int L, int depth, int n_out, int l, float* g_params,
-                            float* Ds, float* As) {
-  const int64_t per = ((n + gridDim.x - 1) / gridDim.x + kDwRows - 1) / kDwRows * kDwRows;
-  const int64_t jb = (int64_t)blockIdx.x * per;
-  const int64_t je = jb + per < n ? jb + per : n;
+                            float* red, InOf in_of) {
+  const int64_t blocks = (n + 31) / 32, per = (blocks + gridDim.x - 1) / gridDim.x;
+  const int64_t b0 = (int64_t)blockIdx.x * per, b1 = b0 + per < blocks ? b0 + per : blocks;
+  if (b0 >= b1) return;  // the whole workgroup
   const int64_t nr = pe_rows(n);
-  dw_layer<IP, OP, INL, OUTL, true>(rows + pe_x_off(l, L, nr), rows + pe_d_off(l, L, depth, n_out, nr), jb, je,
-                                    g_params + pe_param_off(l, L, depth, n_out), Ds, As);
+  dw_layer<OP, IP, OUTL, INL>(rows + pe_d_off(l, L, depth, n_out, nr), rows + pe_x_off(l, L, nr), b0, b1,
+                              g_params + pe_param_off(l, L, depth, n_out), red, in_of);
 }
 
 template <int NOUT>
 __global__ __launch_bounds__(256, 2) void k_pemlp_dw(const float* __restrict__ rows, int64_t n, int L, int depth,
                                                      float* __restrict__ g_params) {
-  __shared__ __align__(16) float Ds[kDwRows * kDwPitch];
-  __shared__ __align__(16) float As[kDwRows * kDwPitch];
+  __shared__ float red[4096];
   constexpr int NOP = NOUT <= 4 ? 4 : 32;
   const int l = blockIdx.y;
   if (l == 0) {
-    pe_dw_layer<64, kPW, 63, kPW>(rows, n, L, depth, NOUT, l, g_params, Ds, As);
+    pe_dw_layer<64, kPW, 63, kPW>(rows, n, L, depth, NOUT, l, g_params, red, [](int i) { return pe_input(i); });
   } else if (l == depth - 1) {
-    pe_dw_layer<kPW, NOP, kPW, NOUT>(rows, n, L, depth, NOUT, l, g_params, Ds, As);
+    pe_dw_layer<kPW, NOP, kPW, NOUT>(rows, n, L, depth, NOUT, l, g_params, red, [](int i) { return i; });
   } else {
-    pe_dw_layer<kPW, kPW, kPW, kPW>(rows, n, L, depth, NOUT, l, g_params, Ds, As);
+    pe_dw_layer<kPW, kPW, kPW, kPW>(rows, n, L, depth, NOUT, l, g_params, red, [](int i) { return i; });
   }
 }
 
@@ -264,9 +280,7 @@ int64_t snisr_pemlp_workspace_size(int64_t n, int32_t L, int32_t depth, int32_t 
 
 namespace {
 int pe_pack(const float* params, int depth, int n_out, float* frag, hipStream_t st) {
-  const int64_t tot = pe_frag_floats(depth, n_out);
-  hipLaunchKernelGGL(k_pack_train_frag, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, params,
-                     pe_param_off(depth, kPL, depth, n_out), frag, kPIn, kPW, depth, 1, n_out);
+  hipLaunchKernelGGL(k_pack_pe, dim3((unsigned)depth), dim3(kPackThreads), 0, st, params, frag, depth, n_out);
   SNISR_LAUNCHED();
   return SNISR_OK;
 }
@@ -285,11 +299,13 @@ int snisr_pemlp_forward(const float* params, const float* points, int64_t n, int
   float* frag = (float*)workspace;
   if (int e = pe_pack(params, depth, n_out, frag, st)) return e;
   const dim3 grid((unsigned)((n + 127) / 128));
+  const int chunks = tr_fwd_chunk(kPIn, kPW, depth, depth);
+  const int64_t bias = tr_bias_off(kPIn, kPW, depth, 0, n_out);
   if (n_out == 28)
-    hipLaunchKernelGGL((k_pemlp_mma<28, false>), grid, dim3(256), 0, st, frag, points, n, (int)depth, slope, out,
+    hipLaunchKernelGGL((k_pemlp_mma<28, false>), grid, dim3(256), 0, st, frag, chunks, bias, points, n, (int)depth, slope, out,
                        nullptr, nullptr);
   else
-    hipLaunchKernelGGL((k_pemlp_mma<4, false>), grid, dim3(256), 0, st, frag, points, n, (int)depth, slope, out,
+    hipLaunchKernelGGL((k_pemlp_mma<4, false>), grid, dim3(256), 0, st, frag, chunks, bias, points, n, (int)depth, slope, out,
                        nullptr, nullptr);
   SNISR_LAUNCHED();
   return SNISR_OK;
@@ -315,11 +331,13 @@ int snisr_pemlp_backward(const float* params, const float* points, int64_t n, in
   float* rows = frag + pe_frag_floats(depth, n_out);
   if (int e = pe_pack(params, depth, n_out, frag, st)) return e;
   const dim3 grid((unsigned)((n + 127) / 128));
+  const int chunks = tr_bwd_chunk(kPIn, kPW, depth, 0, n_out);  // every layer but the first, transposed
+  const int64_t bias = tr_bias_off(kPIn, kPW, depth, 0, n_out);
   if (n_out == 28)
-    hipLaunchKernelGGL((k_pemlp_mma<28, true>), grid, dim3(256), 0, st, (const float*)frag, points, n, (int)depth,
+    hipLaunchKernelGGL((k_pemlp_mma<28, true>), grid, dim3(256), 0, st, (const float*)frag, chunks, bias, points, n, (int)depth,
                        slope, nullptr, g_out, rows);
   else
-    hipLaunchKernelGGL((k_pemlp_mma<4, true>), grid, dim3(256), 0, st, (const float*)frag, points, n, (int)depth,
+    hipLaunchKernelGGL((k_pemlp_mma<4, true>), grid, dim3(256), 0, st, (const float*)frag, chunks, bias, points, n, (int)depth,
                        slope, nullptr, g_out, rows);
   SNISR_LAUNCHED();
   // sample splits of the weight-gradient reduction: about four workgroups per CU over all layers,

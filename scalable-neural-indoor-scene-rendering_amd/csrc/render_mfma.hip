@@ -120,22 +120,25 @@ struct Workspace {
   float4* rec_f;        // [cap] voxel coordinate + weight   (ray-major)
   int2* rec_ti;         // [cap] tile, ray                    (ray-major)
   float4* rgbw;         // [cap] weighted colour of every record (ray-major)
-  int32_t* perm;        // [cap + 64 T] record index in tile order, tile buckets 64-aligned, -1 = padding
+  int32_t* perm;        // [cap + kTrainAlign T] record index in tile order, aligned tile buckets, -1 = padding
   int32_t* tile_count;  // [T]
-  int64_t* tile_start;  // [T+1] 64-aligned bucket starts
+  int64_t* tile_start;  // [T+1] aligned bucket starts
   int64_t* tile_cursor; // [T]
-  uint16_t* enc;        // [n][16] per-ray view encoding in the MFMA operand type (15 values + 0)
+  float* enc;           // [n][16] per-ray view encoding (15 values + 0)
   float4* rec_b;        // [cap] training: interval, T after the sample, clamped sigma, 0
   float4* crec;         // [cap] training: unweighted colour of every record
   float* dsig;          // [cap] training: dL/dsigma of every record
   float* act;           // training: activations/deltas per sorted record (train_act_floats each)
-  float* frag;          // training: per-tile FP32 MFMA weight fragments (forward and transposed)
+  float* frag;          // training: per-tile weight fragments (forward and transposed, train_mma.hpp)
   int64_t cap;
   int32_t n_tiles;
 };
 
 constexpr int kScanItems = 8, kScanBlock = 256, kScanTile = kScanItems * kScanBlock;
 constexpr int kMaxTiles = 4096;  // tile histogram in LDS
+// training: a tile's bucket holds whole workgroups of k_train_mma (4 wavefronts of 32 records), which share the
+// tile's weights through LDS
+constexpr int kTrainAlign = 128;
 
 static inline int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
@@ -153,8 +156,8 @@ static int64_t layout(int64_t n, int64_t cap, int32_t T, uint8_t* base, Workspac
   const int64_t o_tc = off; off = align_up(off + 4 * (int64_t)T, 256);
   const int64_t o_ts = off; off = align_up(off + 8 * ((int64_t)T + 1), 256);
   const int64_t o_cu = off; off = align_up(off + 8 * (int64_t)T, 256);
-  const int64_t o_enc = off; off = align_up(off + 32 * n, 256);
-  const int64_t o_pm = off; off = align_up(off + 4 * (cap + 64 * (int64_t)T), 256);
+  const int64_t o_enc = off; off = align_up(off + 64 * n, 256);
+  const int64_t o_pm = off; off = align_up(off + 4 * (cap + kTrainAlign * (int64_t)T), 256);
   const int64_t o_rf = off; off = align_up(off + 16 * cap, 256);
   const int64_t o_ti = off; off = align_up(off + 8 * cap, 256);
   const int64_t o_rgb = off; off = align_up(off + 16 * cap, 256);
@@ -164,7 +167,7 @@ static int64_t layout(int64_t n, int64_t cap, int32_t T, uint8_t* base, Workspac
     o_rb = off; off = align_up(off + 16 * cap, 256);
     o_cr = off; off = align_up(off + 16 * cap, 256);
     o_ds = off; off = align_up(off + 4 * cap, 256);
-    o_act = off; off = align_up(off + 4 * train_floats * (cap + 64 * (int64_t)T), 256);
+    o_act = off; off = align_up(off + 4 * train_floats * (cap + kTrainAlign * (int64_t)T), 256);
   }
   if (w && base) {
     w->total = reinterpret_cast<int64_t*>(base);
@@ -175,7 +178,7 @@ static int64_t layout(int64_t n, int64_t cap, int32_t T, uint8_t* base, Workspac
     w->tile_count = reinterpret_cast<int32_t*>(base + o_tc);
     w->tile_start = reinterpret_cast<int64_t*>(base + o_ts);
     w->tile_cursor = reinterpret_cast<int64_t*>(base + o_cu);
-    w->enc = reinterpret_cast<uint16_t*>(base + o_enc);
+    w->enc = reinterpret_cast<float*>(base + o_enc);
     w->perm = reinterpret_cast<int32_t*>(base + o_pm);
     w->rec_f = reinterpret_cast<float4*>(base + o_rf);
     w->rec_ti = reinterpret_cast<int2*>(base + o_ti);
@@ -326,7 +329,7 @@ __device__ __forceinline__ void write_encoding(V3 d, int enc_dtype, uint16_t* ou
 // passes took 172 us of the 332 us step of 3,001 rays in one tile, which takes 274 us now)
 template <bool EMIT, int G>  // count the samples, or write their records with the training extras
 __global__ __launch_bounds__(64) void k_march_pass(snisr_scene S, snisr_march_params P, snisr_rays R,
-                                                         snisr_render_out O, Workspace W, int enc_dtype) {
+                                                         snisr_render_out O, Workspace W) {
   const int g = (int)threadIdx.x % G;
   const int64_t i = (int64_t)blockIdx.x * (64 / G) + threadIdx.x / G;
   if (i >= R.n) return;  // whole groups
@@ -362,7 +365,11 @@ __global__ __launch_bounds__(64) void k_march_pass(snisr_scene S, snisr_march_pa
   if (bricks)
     for (int k = m.nbr; k < O.brick_cap; ++k) bricks[k] = -1;
   W.counts[i] = m.nsamp;
-  write_encoding(d, enc_dtype, W.enc + i * 16);
+  float enc[16];
+  view_encoding(d, *reinterpret_cast<float(*)[15]>(&enc));
+  enc[15] = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) store4(W.enc + i * 16 + 4 * q, enc + 4 * q);
   if (O.T) O.T[i] = m.T;
   if (O.n_samples) O.n_samples[i] = m.nsamp;
   if (O.depth) O.depth[i] = m.depth;
@@ -492,7 +499,7 @@ __global__ __launch_bounds__(kScanBlock) void k_tile_scan(Workspace W) {
   int64_t carry = 0;
   for (int start = 0; start < T; start += kScanBlock) {
     const int t = start + threadIdx.x;
-    const int64_t v = t < T ? (int64_t)((W.tile_count[t] + 63) & ~63) : 0;
+    const int64_t v = t < T ? (int64_t)((W.tile_count[t] + kTrainAlign - 1) / kTrainAlign * kTrainAlign) : 0;
     int64_t tot;
     const int64_t ex = block_excl_scan(v, &tot);
     if (t < T) {
@@ -1461,59 +1468,86 @@ __global__ __launch_bounds__(256) void k_train_comp_bwd(Workspace W, int64_t n, 
   }
 }
 
+// dW and db of one layer of one tile over split blockIdx.x of the tile's record blocks.  Bound by reading the
+// rows (3.3 KB per record).  The previous form staged 32-record tiles through LDS for FP32 products and took
+// 2.99 ms for the 3.04M records of the 16-tile step (3.4 TB/s); this one
+// 2.25 ms (4.4 TB/s).
 template <int IN, int WD, int L>
-// two waves per SIMD at least: the 256-register cap keeps the accumulators in VGPRs (AGPR
-// accumulators were copied in and out for every pair and row tile)
 __global__ __launch_bounds__(256, 2) void k_train_dw(Workspace W, int64_t mlp_stride, float* __restrict__ dmlp) {
-  static_assert(WD <= 128 && (IN + 3) / 4 * 4 <= 128, "rows fit the LDS pitch");
-  __shared__ __align__(16) float Ds[kDwRows * kDwPitch];
-  __shared__ __align__(16) float As[kDwRows * kDwPitch];
+  __shared__ float red[4096];
   const int T = W.n_tiles;
   const int tile = blockIdx.y / L, l = blockIdx.y % L;
-  const int64_t NJ = W.cap + 64 * (int64_t)T;
-  const float* A = W.act + NJ * act_a_off(IN, WD, L, l);
-  const float* D = W.act + NJ * act_d_off(IN, WD, L, l);
-  const int64_t j0 = W.tile_start[tile], cnt = W.tile_count[tile];
-  const int64_t per = ((cnt + gridDim.x - 1) / gridDim.x + kDwRows - 1) / kDwRows * kDwRows;
-  const int64_t jb = j0 + (int64_t)blockIdx.x * per;
-  const int64_t je = jb + per < j0 + cnt ? jb + per : j0 + cnt;
+  const int64_t NJ = W.cap + kTrainAlign * (int64_t)T;
+  const int64_t j0 = W.tile_start[tile], blocks = (W.tile_count[tile] + 31) / 32;
+  const int64_t per = (blocks + gridDim.x - 1) / gridDim.x;
+  const int64_t b0 = (int64_t)blockIdx.x * per, b1 = b0 + per < blocks ? b0 + per : blocks;
+  if (b0 >= b1) return;  // the whole workgroup
   float* G = dmlp + (int64_t)tile * mlp_stride + param_w_off(IN, WD, L, l);
-  constexpr int IP0 = in_pad_of(IN, WD, 0);
-  if (l == 0) dw_layer<IP0, WD, IN, WD, true>(A, D, jb, je, G, Ds, As);
-  else if (l == L - 1) dw_layer<WD, 4, WD, 3, true>(A, D, jb, je, G, Ds, As);
-  else dw_layer<WD, WD, WD, WD, true>(A, D, jb, je, G, Ds, As);
+  const float* A = W.act + NJ * act_a_off(IN, WD, L, l) + j0 * in_pad_of(IN, WD, l);
+  const float* D = W.act + NJ * act_d_off(IN, WD, L, l) + j0 * out_pad_of(WD, L, l);
+  if (l == 0) dw_layer<WD, in_pad_of(IN, WD, 0), WD, IN>(D, A, b0, b1, G, red, [](int i) { return i; });
+  else if (l == L - 1) dw_layer<4, WD, 3, WD>(D, A, b0, b1, G, red, [](int i) { return i; });
+  else dw_layer<WD, WD, WD, WD>(D, A, b0, b1, G, red, [](int i) { return i; });
 }
 
-// The FP32 MFMA training MLP helpers (fragment layout, packing, product chains) are in train_mma.hpp.
+// The training MLP's matrix helpers (operand split, fragment layout, packing, staging) are in train_mma.hpp.
+
+__global__ __launch_bounds__(kPackThreads) void k_pack_train(const float* __restrict__ src, int64_t src_stride,
+                                                             float* __restrict__ dst, int in0, int wd, int L) {
+  const int tile = blockIdx.x / L, l = blockIdx.x % L;
+  pack_train_layer(src + (int64_t)tile * src_stride, dst + (int64_t)tile * tr_stride(in0, wd, L, 3), in0, wd, L, l, 3,
+                   [](int row) { return row; });
+}
 
 template <int F, int WD, int L, bool HALF, bool BWD>
 __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays R, Workspace W, float* __restrict__ dsigma,
                                                    float* __restrict__ dfeats) {
-  constexpr int IN = F + 15, NS0 = tr_ns0(IN), NB = WD / 32, NSH = WD / 2;
+  constexpr int IN = F + 15, NS0 = tr_ns0(IN), NB = WD / 32, NKH = WD / 16;
   static_assert(F % 8 == 0 && F <= 32, "feature rows must fill whole 8-row groups of the first block");
   static_assert(WD % 32 == 0 && WD <= 128 && L >= 2 && L <= 8, "MLP shape (one 64-bit ReLU mask per layer)");
-  constexpr int64_t STRIDE = tr_stride(IN, WD, L);
+  static_assert(NS0 % 8 == 0 && in_pad_of(IN, WD, 0) == 2 * NS0, "whole k-chunks of inputs");
+  constexpr int64_t STRIDE = tr_stride(IN, WD, L, 3);
   constexpr int kTrLdsPerWave = 32 * (F + 1) + 2 * 32 * 8 + 32;
-  __shared__ float tr_lds[BWD ? 4 * kTrLdsPerWave : 1];
+  // the weight stream's two buffers; the trilinear adjoint's exchange takes the same memory afterwards
+  constexpr int kLds = BWD && 4 * kTrLdsPerWave * 4 > 2 * kChunkBytes ? 4 * kTrLdsPerWave * 4 : 2 * kChunkBytes;
+  __shared__ __align__(16) uint8_t tr_lds[kLds];
   const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5;
   const int T = W.n_tiles;
-  const int64_t NJ = W.cap + 64 * (int64_t)T;
-  const int64_t j = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 32 + col;
-  int32_t k = -1;
-  if (j < W.tile_start[T]) k = W.perm[j];
-  const bool valid = k >= 0;
-  const uint64_t vm = __ballot(valid);
-  if (vm == 0) return;  // a chunk of padding only (no barriers below)
+  const int64_t NJ = W.cap + kTrainAlign * (int64_t)T;
+  const int64_t groups = W.tile_start[T] / kTrainAlign;
+  const int in_wg = threadIdx.x / 64 * 32 + col;  // this lane's record within the workgroup's group
+  // the next group's record indices and records are loaded while the current group is evaluated
+  int64_t grp = blockIdx.x;
+  int32_t k = -1, lead = -1;
   float4 rf = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   int2 ti = make_int2(0, 0);
-  if (valid) {
-    rf = W.rec_f[k];
-    ti = W.rec_ti[k];
-  }
-  const int tile = __shfl(ti.x, (int)__builtin_ctzll(vm));
+  int tile_v = 0;
+  auto load_index = [&](int64_t g) {
+    k = g < groups ? W.perm[g * kTrainAlign + in_wg] : -1;
+    lead = g < groups ? W.perm[g * kTrainAlign] : -1;  // a group's first record is real
+  };
+  auto load_record = [&] {
+    rf = k >= 0 ? W.rec_f[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    ti = k >= 0 ? W.rec_ti[k] : make_int2(0, 0);
+    tile_v = lead >= 0 ? W.rec_ti[lead].x : 0;
+  };
+  load_index(grp);
+  load_record();
+  for (; grp < groups; grp += gridDim.x) {
+  const int64_t j = grp * kTrainAlign + in_wg;
+  const int32_t kc = k;
+  const float4 rc = rf;
+  const int ray = ti.y;
+  const bool valid = kc >= 0;
+  const int tile = __builtin_amdgcn_readfirstlane(tile_v);  // buckets are aligned: one tile per group
+  const bool any = __ballot(valid) != 0;  // else a wavefront of padding only: it keeps the others' barriers
+  load_index(grp + gridDim.x);
+  FragStream fs;
+  fs.start(W.frag + (int64_t)tile * STRIDE, tr_lds,
+           BWD ? tr_bwd_chunk(IN, WD, L, -1, 3) : tr_fwd_chunk(IN, WD, L, L));
   Corners cn;
   if (valid) {
-    find_corners(S.brick_map + S.tile_brick_base[tile], S.tile_res[tile], v3(rf.x, rf.y, rf.z), cn);
+    find_corners(S.brick_map + S.tile_brick_base[tile], S.tile_res[tile], v3(rc.x, rc.y, rc.z), cn);
   } else {
 #pragma unroll
     for (int q = 0; q < 8; ++q) cn.slot[q] = -1;
@@ -1522,119 +1556,92 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
   uint32_t cmask[8];  // computed ahead of the loads: the masking statements bound scheduling regions
 #pragma unroll
   for (int q = 0; q < 8; ++q) cmask[q] = corner_mask(cn.slot[q] >= 0);
-  // ---- layer-0 inputs: rows tr_row(s, h)
-  float enc[15];
-  {
-    V3 d = v3(1.0f, 0.0f, 0.0f);
-    if (valid) d = normalize_dir(v3(R.dirs[3 * (int64_t)ti.y], R.dirs[3 * (int64_t)ti.y + 1], R.dirs[3 * (int64_t)ti.y + 2]));
-    view_encoding(d, enc);
-  }
+  // ---- layer-0 inputs, rows tr_row(s, h): features, then the ray's view encoding (16 floats per ray)
   float x0[NS0];
   gather_rows<F, HALF>(S.feats, cn, cmask, h, x0);
+  const float* enc = W.enc + 16 * (int64_t)ray;
 #pragma unroll
   for (int g = F / 8; g < NS0 / 4; ++g) {
-    const int base = 32 * (g / 4) + 8 * (g % 4);  // first row of the 8-row group (lane half 0)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int e0 = base - F + t, e1 = e0 + 4;  // view-encoding index for lane half 0 / 1
-      const float v0 = e0 < 15 ? enc[e0 < 15 ? e0 : 0] : 0.0f;
-      const float v1 = e1 < 15 ? enc[e1 < 15 ? e1 : 0] : 0.0f;
-      x0[4 * g + t] = h ? v1 : v0;
-    }
+    float4 e = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (valid) e = *reinterpret_cast<const float4*>(enc + 8 * (g - F / 8) + 4 * h);
+    x0[4 * g] = e.x;
+    x0[4 * g + 1] = e.y;
+    x0[4 * g + 2] = e.z;
+    x0[4 * g + 3] = e.w;
   }
-  const float* P = W.frag + (int64_t)tile * STRIDE;
+  const float* bias = W.frag + (int64_t)tile * STRIDE + tr_bias_off(IN, WD, L, 0, 3);
+  const float* winv = W.frag + (int64_t)tile * STRIDE + tr_scale_off(IN, WD, L, 3);
   float* act = W.act;
-  if (BWD && valid) {
-    // rows in the lane layout of the weight-gradient reduction: group g of this wavefront's 32
-    // records is one contiguous 1 KB store
-    float* A0 = act + NJ * act_a_off(IN, WD, L, 0) + (j - col) * in_pad_of(IN, WD, 0) + 4 * lane;
-#pragma unroll
-    for (int g = 0; g < NS0 / 4; ++g) store4(A0 + 256 * g, x0 + 4 * g);
-  }
+  // rows of this wavefront's 32-record block, as the weight-gradient reduction reads them (padding records
+  // have zero deltas)
+  if (BWD && any) store_rows<in_pad_of(IN, WD, 0), NS0 / 4>(act + NJ * act_a_off(IN, WD, L, 0) + (j - col) * in_pad_of(IN, WD, 0), x0, lane);
   // ---- forward: hidden layers (ReLU), masks of every hidden input for the backward
   float a[NB * 16];
   uint64_t mask[L];
-  mma_blocks<NS0, NB>(
-      P + tr_fwd_off(IN, WD, L, 0), x0, lane, [&](int ob) { return bias_block(P + tr_bias_off(IN, WD, L, 0), ob, h); },
-      [&](int ob, const f32x16& acc) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) a[ob * 16 + r] = acc[r] > 0.0f ? acc[r] : 0.0f;
-      });
+  auto relu = [&](int r, float v) { a[r] = v > 0.0f ? v : 0.0f; };
+  stream_layer<NS0 / 8, NB>(fs, x0, lane, winv[0], bias, relu);
 #pragma unroll
   for (int l = 1; l < L; ++l) {
+    bias += 32 * NB;
     mask[l] = 0;
 #pragma unroll
     for (int r = 0; r < NB * 16; ++r) mask[l] |= (uint64_t)(a[r] > 0.0f) << (r & 63);
-    if (BWD && valid) {
-      float* Al = act + NJ * act_a_off(IN, WD, L, l) + (j - col) * WD + 4 * lane;
+    if (BWD && any) store_rows<WD, NB * 4>(act + NJ * act_a_off(IN, WD, L, l) + (j - col) * WD, a, lane);
+    if (l < L - 1) {
+      float y[NB * 16];
+      stream_layer<NKH, NB>(fs, a, lane, winv[l], bias, [&](int r, float v) { y[r] = v > 0.0f ? v : 0.0f; });
 #pragma unroll
-      for (int g = 0; g < NB * 4; ++g) store4(Al + 256 * g, a + 4 * g);
+      for (int r = 0; r < NB * 16; ++r) a[r] = y[r];
     }
-    if (l == L - 1) break;
-    float b[NB * 16];
-    mma_blocks<NSH, NB>(
-        P + tr_fwd_off(IN, WD, L, l), a, lane, [&](int ob) { return bias_block(P + tr_bias_off(IN, WD, L, l), ob, h); },
-        [&](int ob, const f32x16& acc) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) b[ob * 16 + r] = acc[r] > 0.0f ? acc[r] : 0.0f;
-        });
-#pragma unroll
-    for (int r = 0; r < NB * 16; ++r) a[r] = b[r];
   }
+  load_record();  // of the next group
   // ---- output layer: rows 0..2 (lane half 0, registers 0..2)
-  f32x16 z = bias_block(P + tr_bias_off(IN, WD, L, L - 1), 0, h);
-  z = mma_f32_chain<NSH>(P + tr_fwd_off(IN, WD, L, L - 1), a, z, lane);
+  float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
+  stream_layer<NKH, 1>(fs, a, lane, winv[L - 1], bias, [&](int r, float v) {
+    if (r == 0) c0 = sigmoid_cw(v);
+    if (r == 1) c1 = sigmoid_cw(v);
+    if (r == 2) c2 = sigmoid_cw(v);
+  });
   if (!BWD) {
     if (valid && h == 0) {
-      const float c0 = sigmoid_cw(z[0]), c1 = sigmoid_cw(z[1]), c2 = sigmoid_cw(z[2]);
-      W.crec[k] = make_float4(c0, c1, c2, 0.0f);
-      W.rgbw[k] = make_float4(rf.w * c0, rf.w * c1, rf.w * c2, 0.0f);
+      W.crec[kc] = make_float4(c0, c1, c2, 0.0f);
+      W.rgbw[kc] = make_float4(rc.w * c0, rc.w * c1, rc.w * c2, 0.0f);
     }
-    return;
+    __syncthreads();  // the weight stream's buffers are free for the next group
+    continue;
   }
   // ---- output delta from dL/dc (written into rgbw by the compositing adjoint)
-  float dout[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  float dout[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   if (valid && h == 0) {
-    const float4 dc = W.rgbw[k];
-    const float c0 = sigmoid_cw(z[0]), c1 = sigmoid_cw(z[1]), c2 = sigmoid_cw(z[2]);
+    const float4 dc = W.rgbw[kc];
     dout[0] = dc.x * c0 * (1.0f - c0);
     dout[1] = dc.y * c1 * (1.0f - c1);
     dout[2] = dc.z * c2 * (1.0f - c2);
-    store4(act + NJ * act_d_off(IN, WD, L, L - 1) + j * 4, dout);
   }
+  if (any) store_rows<4, 1>(act + NJ * act_d_off(IN, WD, L, L - 1) + (j - col) * 4, dout, lane);
   // ---- backpropagate: d_{l-1} = mask_l (W_l^T d_l)
   float d[NB * 16];
-  mma_blocks<4, NB>(
-      P + tr_bwd_off(IN, WD, L, L - 1), dout, lane, [&](int) { return f32x16{}; },
-      [&](int ib, const f32x16& acc) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) d[ib * 16 + r] = ((mask[L - 1] >> ((ib * 16 + r) & 63)) & 1) ? acc[r] : 0.0f;
-      });
+  stream_layer<1, NB>(fs, dout, lane, winv[L - 1], nullptr,
+                      [&](int r, float v) { d[r] = ((mask[L - 1] >> (r & 63)) & 1) ? v : 0.0f; });
 #pragma unroll
   for (int l = L - 2; l >= 0; --l) {
-    if (valid) {
-      float* Dl = act + NJ * act_d_off(IN, WD, L, l) + (j - col) * WD + 4 * lane;
+    if (any) store_rows<WD, NB * 4>(act + NJ * act_d_off(IN, WD, L, l) + (j - col) * WD, d, lane);
+    if (l > 0) {
+      float e[NB * 16];
+      stream_layer<NKH, NB>(fs, d, lane, winv[l], nullptr,
+                            [&](int r, float v) { e[r] = ((mask[l] >> (r & 63)) & 1) ? v : 0.0f; });
 #pragma unroll
-      for (int g = 0; g < NB * 4; ++g) store4(Dl + 256 * g, d + 4 * g);
+      for (int r = 0; r < NB * 16; ++r) d[r] = e[r];
     }
-    if (l == 0) break;
-    float e[NB * 16];
-    mma_blocks<NSH, NB>(
-        P + tr_bwd_off(IN, WD, L, l), d, lane, [&](int) { return f32x16{}; },
-        [&](int ib, const f32x16& acc) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) e[ib * 16 + r] = ((mask[l] >> ((ib * 16 + r) & 63)) & 1) ? acc[r] : 0.0f;
-        });
-#pragma unroll
-    for (int r = 0; r < NB * 16; ++r) d[r] = e[r];
   }
   // ---- dL/d(features): rows 0..F-1 of W_0^T d_0
-  f32x16 df = {};
-  df = mma_f32_chain<NSH>(P + tr_bwd_off(IN, WD, L, 0), d, df, lane);
+  float df[16];
+  stream_layer<NKH, 1>(fs, d, lane, winv[0], nullptr, [&](int r, float v) { df[r] = v; });
+  __syncthreads();  // the weight stream's buffers become the exchange area
   // ---- trilinear adjoint.  The wave's 32 records go through LDS so that each atomic instruction
   // covers whole feature rows (64 / F records x F contiguous features) instead of 64 scattered
   // values; padding records have no corners.
-  float* dfl = tr_lds + (threadIdx.x >> 6) * kTrLdsPerWave;  // [32][F + 1] feature gradients
+  float* dfl = reinterpret_cast<float*>(tr_lds) + (threadIdx.x >> 6) * kTrLdsPerWave;  // [32][F + 1] feature gradients
   float* wl = dfl + 32 * (F + 1);                             // [32][8] corner weights
   int* sl = reinterpret_cast<int*>(wl + 32 * 8);              // [32][8] corner slots
   float* gl = wl + 2 * 32 * 8;                                // [32] dL/dsigma
@@ -1649,7 +1656,7 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
       wl[col * 8 + q] = wx[q & 1] * wy[(q >> 1) & 1] * wz[q >> 2];
       sl[col * 8 + q] = cn.slot[q];
     }
-    gl[col] = valid ? W.dsig[k] : 0.0f;
+    gl[col] = valid ? W.dsig[kc] : 0.0f;
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1708,6 +1715,8 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
       }
     }
     if (cur >= 0 && run != 0.0f) atomicAdd(&dsigma[cur], run);
+  }
+  __syncthreads();  // the exchange area becomes the next group's weight buffers
   }
 }
 
@@ -2024,8 +2033,15 @@ static int dw_splits(int64_t tile_layers) {
   return (int)(s < 1 ? 1 : (s > 128 ? 128 : s));
 }
 
+// workgroups of k_train_mma: those that are resident together (two per CU at width 128, else four), each
+// walking the 128-record groups of the sorted order
+static unsigned train_groups(int64_t cap, int n_tiles, int width) {
+  const int64_t most = (cap + kTrainAlign * (int64_t)n_tiles) / kTrainAlign, resident = (width > 64 ? 2 : 4) * (int64_t)device_cus();
+  return (unsigned)(most < resident ? most : resident);
+}
+
 static int64_t train_frag_floats(const snisr_scene* s) {
-  return (int64_t)s->n_tiles * tr_stride(s->mlp_in, s->mlp_width, s->mlp_layers);
+  return (int64_t)s->n_tiles * tr_stride(s->mlp_in, s->mlp_width, s->mlp_layers, 3);
 }
 
 int64_t snisr_train_workspace_size(const snisr_scene* scene, int64_t n, int64_t sample_capacity) {
@@ -2087,7 +2103,7 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   const dim3 mgrid((unsigned)((n * lanes + 63) / 64));
 #define SNISR_MARCH_PASS(EMIT_, G_)                                                                                   \
   if (lanes == G_)                                                                                                    \
-    hipLaunchKernelGGL((k_march_pass<EMIT_, G_>), mgrid, dim3(64), 0, st, *scene, *params, *rays, *out, W, (int)SNISR_F16);
+    hipLaunchKernelGGL((k_march_pass<EMIT_, G_>), mgrid, dim3(64), 0, st, *scene, *params, *rays, *out, W);
   SNISR_MARCH_PASS(false, 8)
   SNISR_MARCH_PASS(false, 4)
   SNISR_MARCH_PASS(false, 2)
@@ -2113,12 +2129,11 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   SNISR_LAUNCHED();
   SNISR_HIP(stage_event(out, 1, st));
   {  // this step's weights as FP32 MFMA fragments (the backward reads the same copy)
-    const int64_t tot = train_frag_floats(scene);
-    hipLaunchKernelGGL(k_pack_train_frag, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, scene->mlp_params,
-                       scene->mlp_stride, W.frag, scene->mlp_in, WD, L, scene->n_tiles, 3);
+    hipLaunchKernelGGL(k_pack_train, dim3((unsigned)(scene->n_tiles * L)), dim3(kPackThreads), 0, st, scene->mlp_params,
+                       scene->mlp_stride, W.frag, scene->mlp_in, WD, L);
     SNISR_LAUNCHED();
   }
-  const dim3 jgrid((unsigned)((cap + 64 * (int64_t)scene->n_tiles + 127) / 128));
+  const dim3 jgrid(train_groups(cap, scene->n_tiles, WD));
 #define SNISR_FWD(F_, W_, L_, H_)                                                                      \
   if (F == F_ && WD == W_ && L == L_ && half == H_)                                                      \
     hipLaunchKernelGGL((k_train_mma<F_, W_, L_, H_, false>), jgrid, dim3(256), 0, st, *scene, *rays, W, \
@@ -2169,7 +2184,7 @@ int snisr_train_backward(const snisr_scene* scene, const snisr_march_params* par
   hipLaunchKernelGGL(k_train_comp_bwd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, W, n, grad_rgb);
   SNISR_LAUNCHED();
   SNISR_HIP(stage_event(&ev, 1, st));
-  const dim3 jgrid((unsigned)((cap + 64 * (int64_t)scene->n_tiles + 127) / 128));
+  const dim3 jgrid(train_groups(cap, scene->n_tiles, WD));
   bool ok = false;
 #define SNISR_BWD(F_, W_, L_, H_)                                                                            \
   if (F == F_ && WD == W_ && L == L_ && half == H_) {                                                        \

@@ -1,125 +1,128 @@
-// Weight-gradient reduction shared by the FP32 training kernels: dW += D^T A and db += sum D over
-// a range of stored per-sample rows, on v_mfma_f32_32x32x2_f32.
+// Weight-gradient reduction shared by the FP32 training kernels: dW += D^T A and db += sum D over a range
+// of stored 32-record blocks (train_mma.hpp's row layout), the records as the K dimension.
 #pragma once
 
-#include "mfma_ops.hpp"
+#include "train_mma.hpp"
 
 namespace snisr {
 
-// dW_l[o][i] += sum_j D_l[j][o] A_l[j][i] and db_l[o] += sum_j D_l[j][o] over one split of one tile's
-// sorted records, on v_mfma_f32_32x32x2_f32 with the records as the K dimension.  A workgroup owns
-// every (out-block, in-block) pair of the layer (at most 16 pairs of 32 x 32; wave w takes pairs
-// w, w + 4, ...) and walks its records in tiles of 32 staged through LDS: the A operand of step s
-// is D rows 2s + h at columns ob*32 + c, the B operand A rows 2s + h at columns ib*32 + c.  Rows are
-// padded to 160 floats so that the two lane halves read disjoint banks.  The next tile's rows are
-// loaded into registers while the current tile's products run.
-//
-// Row layouts: with LANE false the rows are per record ([record][feature], pitch IP / OP); with LANE
-// true each 32-record block (blocks start at multiples of 32) is stored in the order the training
-// kernel's lanes hold it, feature group g (256 floats) = lane l's four features
-// 32 (g / 4) + 8 (g % 4) + 4 (l / 32) .. + 3 of record l % 32, so that the kernel writes every
-// group with one 1 KB wavefront store; a pitch of 4 is the same in both layouts.
-constexpr int kDwRows = 32, kDwPitch = 160;
-// float offset of (record, feature f, a multiple of 4) inside a 32-record block in the lane layout
-__device__ __forceinline__ int lane_off(int rec, int f) {
-  return 256 * (4 * (f >> 5) + ((f >> 3) & 3)) + 4 * (rec + 32 * ((f >> 2) & 1));
-}
-template <int IP, int OP, int INL, int OUTL, bool LANE = false>  // padded row widths, real in / out sizes
-__device__ __forceinline__ void dw_layer(const float* __restrict__ A, const float* __restrict__ D, int64_t jb,
-                                         int64_t je, float* __restrict__ G, float* Ds, float* As) {
-  static_assert(!LANE || ((IP % 8 == 0 || IP == 4) && (OP % 8 == 0 || OP == 4)), "lane layout pitches");
-  constexpr int IP4 = IP / 4, OP4 = OP / 4;
-  constexpr int ND = (kDwRows * OP4 + 255) / 256, NA = (kDwRows * IP4 + 255) / 256;
-  constexpr int NIB = (INL + 31) / 32, NOB = (OUTL + 31) / 32, NPAIR = NIB * NOB;
-  static_assert(NPAIR <= 16, "at most 4 pairs per wave");
-  static_assert(2 * OP <= 256, "two threads per output column");
-  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
-  f32x16 acc[4];
+// One wavefront's share of a layer: NA output blocks from ob0 and NB input blocks from ib0 over the record
+// blocks j0, j0 + dj, ... < j1.  A lane of an operand is a feature and its k slots are records, so both
+// operands come straight from memory in 1 KB loads (no LDS, no barriers), the next half block's loads in
+// flight while the current one is split into its BF16 parts and multiplied.
+// OW / IW: row widths, OUTL / INL: real outputs and inputs; in_of: the input stored at a row.
+// With `red` (NA NB 1024 floats of LDS) the workgroup's wavefronts hold the same blocks: they are added there
+// first and only the sums go out.
+template <int OW, int IW, int OUTL, int INL, int NA, int NB, class InOf>
+__device__ __forceinline__ void dw_wave(const float* __restrict__ D, const float* __restrict__ A, int64_t j0, int64_t j1,
+                                        int64_t dj, int ob0, int ib0, float* __restrict__ G, InOf in_of, float* red = nullptr) {
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  f32x16 acc[NA][NB];
+  float db[NA];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) acc[q] = f32x16{};
-  float accb = 0.0f;
-  float4 rd[ND], ra[NA];
-  // thread q moves float4 (record q / P4, features 4 (q % P4) ..) of the 32-record tile, so that the
-  // LDS stores below are conflict-free; in the lane layout its global load then reads 16 bytes of
-  // a line that the workgroup's other loads of the tile complete
-  auto fetch = [&](int64_t r0) {
+  for (int i = 0; i < NA; ++i) {
+    db[i] = 0.0f;
 #pragma unroll
-    for (int u = 0; u < ND; ++u) {
-      const int q = threadIdx.x + 256 * u, rr = q / OP4, cc = 4 * (q % OP4);
-      rd[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (q < kDwRows * OP4 && r0 + rr < je)
-        rd[u] = *reinterpret_cast<const float4*>(D + r0 * OP + (LANE ? lane_off(rr, cc) : rr * OP + cc));
-    }
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x16{};
+  }
+  // values of k-chunk kc (records 16 kc .. +15) of block b of a W-wide row: two pieces of four records
+  float nd[NA][8], na[NB][8];
+  auto load = [&](const float* rows, int64_t blk, int W, int b, int kc, float (&v)[8]) {
+    const int w = W - 32 * b < 32 ? W - 32 * b : 32;
+    const float* p = rows + blk * 32 * W + 1024 * b + 4 * c;
 #pragma unroll
-    for (int u = 0; u < NA; ++u) {
-      const int q = threadIdx.x + 256 * u, rr = q / IP4, cc = 4 * (q % IP4);
-      ra[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (q < kDwRows * IP4 && r0 + rr < je)
-        ra[u] = *reinterpret_cast<const float4*>(A + r0 * IP + (LANE ? lane_off(rr, cc) : rr * IP + cc));
+    for (int u = 0; u < 2; ++u) {
+      float4 t = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (c < w) t = *reinterpret_cast<const float4*>(p + 4 * w * (4 * kc + 2 * u + h));
+      v[4 * u] = t.x;
+      v[4 * u + 1] = t.y;
+      v[4 * u + 2] = t.z;
+      v[4 * u + 3] = t.w;
     }
   };
-  if (jb < je) fetch(jb);
-  for (int64_t r0 = jb; r0 < je; r0 += kDwRows) {
-    __syncthreads();  // the previous tile's reads of Ds / As are done
+  auto fetch = [&](int64_t blk, int kc) {
 #pragma unroll
-    for (int u = 0; u < ND; ++u) {
-      const int q = threadIdx.x + 256 * u;
-      if (q < kDwRows * OP4) *reinterpret_cast<float4*>(Ds + (q / OP4) * kDwPitch + 4 * (q % OP4)) = rd[u];
-    }
+    for (int i = 0; i < NA; ++i) load(D, blk, OW, ob0 + i, kc, nd[i]);
 #pragma unroll
-    for (int u = 0; u < NA; ++u) {
-      const int q = threadIdx.x + 256 * u;
-      if (q < kDwRows * IP4) *reinterpret_cast<float4*>(As + (q / IP4) * kDwPitch + 4 * (q % IP4)) = ra[u];
-    }
-    __syncthreads();
-    if (r0 + kDwRows < je) fetch(r0 + kDwRows);
-    // db: thread t < 2 OP sums rows (t / OP) * 16 .. + 15 of column t % OP, four independent
-    // partial sums so that the LDS reads do not wait on each other
-    if (threadIdx.x < 2 * OP) {
-      const int col = threadIdx.x % OP, r0h = (threadIdx.x / OP) * (kDwRows / 2);
-      float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < NB; ++j) load(A, blk, IW, ib0 + j, kc, na[j]);
+  };
+  if (j0 < j1) fetch(j0, 0);
+#pragma unroll 1
+  for (int64_t blk = j0; blk < j1; blk += dj) {
 #pragma unroll
-      for (int rr = 0; rr < kDwRows / 2; ++rr) part[rr & 3] += Ds[(r0h + rr) * kDwPitch + col];
-      accb += (part[0] + part[1]) + (part[2] + part[3]);
-    }
-    // the 16 steps' operands of the wave's next pair are read from LDS while the current pair's
-    // products run (a ring of two operand sets), so no product waits on its own LDS read
-    float xs[2][kDwRows / 2], ys[2][kDwRows / 2];
-    auto load_pair = [&](int p, float (&x)[kDwRows / 2], float (&y)[kDwRows / 2]) {
-      const int ob = p / NIB, ib = p % NIB;
+    for (int kc = 0; kc < 2; ++kc) {
+      Split8 a[NA], b[NB];
 #pragma unroll
-      for (int st = 0; st < kDwRows / 2; ++st) {
-        x[st] = Ds[(2 * st + h) * kDwPitch + ob * 32 + c];
-        y[st] = As[(2 * st + h) * kDwPitch + ib * 32 + c];
+      for (int i = 0; i < NA; ++i) {
+        a[i] = split8(nd[i]);
+        db[i] += ((nd[i][0] + nd[i][1]) + (nd[i][2] + nd[i][3])) + ((nd[i][4] + nd[i][5]) + (nd[i][6] + nd[i][7]));
       }
-    };
-    if (wv < NPAIR) load_pair(wv, xs[0], ys[0]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int p = wv + 4 * q;
-      if (p < NPAIR) {  // wave-uniform
-        if (q + 1 < 4 && p + 4 < NPAIR) load_pair(p + 4, xs[(q + 1) & 1], ys[(q + 1) & 1]);
-        f32x16 a = acc[q];
+      for (int j = 0; j < NB; ++j) b[j] = split8(na[j]);
+      if (kc == 0) fetch(blk, 1);
+      else if (blk + dj < j1) fetch(blk + dj, 0);
+      mma_split<NA, NB>(a, b, acc);
+    }
+  }
+  const int wv = threadIdx.x >> 6;
+  if (red) {
+    for (int w = 1; w < 4; ++w) {  // wavefront w hands its sums to wavefront 0
+      __syncthreads();
+      if (wv == w) {
 #pragma unroll
-        for (int st = 0; st < kDwRows / 2; ++st) a = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[q & 1][st], ys[q & 1][st], a, 0, 0, 0);
-        acc[q] = a;
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) red[((i * NB + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+      }
+      __syncthreads();
+      if (wv == 0) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] += red[((i * NB + j) * 16 + r) * 64 + lane];
       }
     }
   }
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int p = wv + 4 * q;
-    if (p >= NPAIR) break;
-    const int ob = p / NIB, ib = p % NIB;
-    const int i = ib * 32 + c;
+  for (int i = 0; i < NA; ++i) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int o = ob * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-      if (o < OUTL && i < INL && acc[q][r] != 0.0f) atomicAdd(&G[(int64_t)o * INL + i], acc[q][r]);
+    for (int j = 0; j < NB; ++j) {
+      if (red && wv) break;
+      const int in = in_of(32 * (ib0 + j) + c);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int o = 32 * (ob0 + i) + 8 * (r / 4) + 4 * h + (r % 4);
+        if (o < OUTL && in < INL && acc[i][j][r] != 0.0f) atomicAdd(&G[(int64_t)o * INL + in], acc[i][j][r]);
+      }
     }
+    const float s = db[i] + __shfl_xor(db[i], 32);
+    const int o = 32 * (ob0 + i) + c;
+    if (ib0 == 0 && h == 0 && o < OUTL && s != 0.0f) atomicAdd(&G[(int64_t)OUTL * INL + o], s);
   }
-  if (threadIdx.x < 2 * OP && threadIdx.x % OP < OUTL && accb != 0.0f)
-    atomicAdd(&G[(int64_t)OUTL * INL + threadIdx.x % OP], accb);
+}
+
+// dW_l[o][i] += sum_j D_l[j][o] A_l[j][i] and db_l[o] += sum_j D_l[j][o] over the record blocks [j0, j1) of a
+// four-wavefront workgroup.  A layer of at most 2 x 2 blocks gives every wavefront all of them over every
+// fourth record block (red: 4096 floats of LDS); a larger one gives each wavefront a part of the blocks over all records.
+template <int OW, int IW, int OUTL, int INL, class InOf>
+__device__ __forceinline__ void dw_layer(const float* __restrict__ D, const float* __restrict__ A, int64_t j0, int64_t j1,
+                                         float* __restrict__ G, float* red, InOf in_of) {
+  constexpr int NOB = (OUTL + 31) / 32, NIB = (INL + 31) / 32;
+  const int wv = threadIdx.x >> 6;
+  if constexpr (NOB <= 2 && NIB <= 2) {
+    dw_wave<OW, IW, OUTL, INL, NOB, NIB>(D, A, j0 + wv, j1, 4, 0, 0, G, in_of, red);
+  } else if constexpr (NOB == 4 && NIB == 4) {
+    dw_wave<OW, IW, OUTL, INL, 2, 2>(D, A, j0, j1, 1, 2 * (wv >> 1), 2 * (wv & 1), G, in_of);
+  } else if constexpr (NOB == 4 && NIB == 2) {
+    dw_wave<OW, IW, OUTL, INL, 2, 1>(D, A, j0, j1, 1, 2 * (wv >> 1), wv & 1, G, in_of);
+  } else {
+    static_assert(NOB == 1 && NIB == 4, "layer shapes of the training MLPs");
+    dw_wave<OW, IW, OUTL, INL, 1, 2>(D, A, j0 + (wv >> 1), j1, 2, 0, 2 * (wv & 1), G, in_of);
+  }
 }
 
 }  // namespace snisr

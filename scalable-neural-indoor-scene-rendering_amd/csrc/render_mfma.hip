@@ -699,6 +699,38 @@ struct RunList {
   __device__ __forceinline__ void store(int4* dst) const { *dst = make_int4(v0, v1, v2, v3); }
 };
 
+// Records staged per lane in LDS until eight are there, 128 bytes of a ray's slots (lines written piecemeal by many
+// rays in flight would leave L2 partly written, several times over).  flush_full() writes the lanes that hold eight:
+// eight lanes take one ray's records, so that one store serves up to eight rays.  Called by lanes that may have
+// diverged; the active ones share the work.  The marches of unrelated rays are bound by the address path of the L1
+// (87% busy, a wavefront's load or store takes it 16 cycles and more however few lanes are active), and with each
+// full lane storing its own eight, almost every sample step issued eight stores for one or two lanes.
+struct RecordStage {
+  float4 rec[8][64];   // record j of lane l
+  float4* to[64];      // destination of the r-th full lane
+  int from[64];        // its lane
+};
+__device__ __forceinline__ void flush_full(RecordStage& st, bool full, float4* dst) {
+  const uint64_t fm = __builtin_amdgcn_ballot_w64(full);
+  if (!fm) return;
+  const uint64_t am = __builtin_amdgcn_ballot_w64(true);
+  const int lane = threadIdx.x & 63;
+  const uint64_t below = (1ull << lane) - 1;
+  if (full) {
+    const int r = __builtin_popcountll(fm & below);
+    st.to[r] = dst;
+    st.from[r] = lane;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int n = 8 * __builtin_popcountll(fm), helpers = __builtin_popcountll(am);
+  for (int p = __builtin_popcountll(am & below); p < n; p += helpers) st.to[p >> 3][p & 7] = st.rec[p & 7][st.from[p >> 3]];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // One wavefront per 64 rays: march each ray once, writing its records (voxel coordinate + weight,
 // tile) at its own slots, its sample count, T, depth and view encoding; per-wave totals feed the
 // header (sample total, largest count, overflow when a ray has more samples than slots).
@@ -781,8 +813,10 @@ __global__ __launch_bounds__(256) void k_ray_enc(snisr_rays R, RenderWs W, int e
 
 // The march of arbitrary rays (no pixel packets, or a ray schedule) as a queue: a wavefront's lanes
 // take rays (thread indices tid0 .. tid1 - 1, ray = order[tid] or tid) from a per-chunk counter and,
-// when a quarter of the lanes have finished theirs, take new ones together, so that a wavefront is
-// not held by its longest ray while most lanes idle.  Each ray is marched exactly as by
+// when a quarter of the lanes have finished theirs, write their results and take new ones together, so that a
+// wavefront is not held by its longest ray while most lanes idle.  1.0M unrelated rays over 27 tiles: 1660 -> 1465 us
+// with the results and full record lines written together; more wavefronts per SIMD (128 registers: +16%), a
+// refill at an eighth (+8%) and sample steps held back for 24 lanes (+4%) were slower.  Each ray is marched exactly as by
 // march_ray (FlatMarch: same steps, same records), only the lanes that run it change.  The grid is sized
 // to the device's resident wavefronts; every wavefront ends once the counter passes tid1 and its
 // lanes' rays are done.
@@ -790,7 +824,7 @@ constexpr int kRefillQuorum = 4;
 __global__ __launch_bounds__(64) void k_march_queue(snisr_scene S, snisr_march_params P, snisr_rays R,
                                                     snisr_render_out O, RenderWs W, const int32_t* __restrict__ order,
                                                     int64_t tid0, int64_t tid1) {
-  __shared__ float4 rbuf[8][64];   // records staged per lane, written 8 at a time (see k_march_render)
+  __shared__ RecordStage stage;
   const int lane = threadIdx.x;
   const int cpr = W.cpr;
   FlatMarch m;
@@ -800,6 +834,7 @@ __global__ __launch_bounds__(64) void k_march_queue(snisr_scene S, snisr_march_p
   int kr = 0, run_tile = -1, run_start = 0;
   RunList rl;
   rl.reset();
+  bool full = false;  // this lane's eight staged records wait to be written
   int32_t* bricks = nullptr;
   int64_t sum = 0;
   int mx = 0;
@@ -807,7 +842,7 @@ __global__ __launch_bounds__(64) void k_march_queue(snisr_scene S, snisr_march_p
     float4* dst = W.rec_f + slot0 + base;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (j < cnt) dst[j] = rbuf[j][lane];
+      if (j < cnt) dst[j] = stage.rec[j][lane];
   };
   auto on_sample = [&](int tile, const V3& f, const Corners&, float w, float, float, float) {
     if (kr < cpr) {
@@ -816,61 +851,66 @@ __global__ __launch_bounds__(64) void k_march_queue(snisr_scene S, snisr_march_p
         run_tile = tile;
         run_start = kr;
       }
-      const int j = kr & 7;
-      rbuf[j][lane] = make_float4(f.x, f.y, f.z, w);
-      if (j == 7) flush(kr - 7, 8);
+      stage.rec[kr & 7][lane] = make_float4(f.x, f.y, f.z, w);
+      full = (kr & 7) == 7;
     }
     ++kr;
   };
   while (true) {
-    if (has && m.phase == FlatMarch::kDone) {  // finish this lane's ray
-      const int nrec = min(kr, cpr);
-      if (nrec & 7) flush(nrec & ~7, nrec & 7);
-      if (run_tile >= 0) rl.add(run_tile | ((nrec - run_start) << 16), W.rec_t + slot0);
-      rl.store(W.runs4 + i);
-      if (bricks)
-        for (int b = m.nbr; b < O.brick_cap; ++b) bricks[b] = -1;
-      W.counts[i] = m.nsamp;
-      if (O.T) O.T[i] = m.T;
-      if (O.n_samples) O.n_samples[i] = m.nsamp;
-      if (O.depth) O.depth[i] = m.depth;
-      sum += m.nsamp;
-      mx = m.nsamp > mx ? m.nsamp : mx;
-      has = false;
-    }
-    const uint64_t idle = __builtin_amdgcn_ballot_w64(!has && more);
-    const uint64_t busy = __builtin_amdgcn_ballot_w64(has);
+    const bool done = has && m.phase == FlatMarch::kDone;
+    const uint64_t idle = __builtin_amdgcn_ballot_w64(done || (!has && more));
+    const uint64_t busy = __builtin_amdgcn_ballot_w64(has && !done);
     if (idle && (busy == 0 || kRefillQuorum * __builtin_popcountll(idle) >= 64)) {
-      const int first = (int)__builtin_ctzll(idle);
-      unsigned long long base = 0;
-      if (lane == first) base = atomicAdd(W.cursor, (unsigned long long)__builtin_popcountll(idle));
-      base = ((unsigned long long)(uint32_t)__shfl((int)(uint32_t)(base >> 32), first) << 32) |
-             (uint32_t)__shfl((int)(uint32_t)base, first);
-      if (!has && more) {
-        const int64_t t = tid0 + (int64_t)base + __builtin_popcountll(idle & ((1ull << lane) - 1));
-        if (t < tid1) {
-          i = order ? (int64_t)order[t] : t;
-          const float* og = R.origins + i * R.origin_stride;
-          const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
-          m.init(S, P, v3(og[0], og[1], og[2]), d, R.t_hit ? R.t_hit[i] : __builtin_inff(),
-                 R.visited ? R.visited + i * P.max_tiles : nullptr);
-          slot0 = i * (int64_t)cpr;
-          kr = 0;
-          run_tile = -1;
-          run_start = 0;
-          rl.reset();
-          bricks = O.bricks ? O.bricks + i * O.brick_cap : nullptr;
-          has = true;
-        } else {
-          more = false;
+      if (done) {  // finish this lane's ray
+        const int nrec = min(kr, cpr);
+        if (nrec & 7) flush(nrec & ~7, nrec & 7);
+        if (run_tile >= 0) rl.add(run_tile | ((nrec - run_start) << 16), W.rec_t + slot0);
+        rl.store(W.runs4 + i);
+        if (bricks)
+          for (int b = m.nbr; b < O.brick_cap; ++b) bricks[b] = -1;
+        W.counts[i] = m.nsamp;
+        if (O.T) O.T[i] = m.T;
+        if (O.n_samples) O.n_samples[i] = m.nsamp;
+        if (O.depth) O.depth[i] = m.depth;
+        sum += m.nsamp;
+        mx = m.nsamp > mx ? m.nsamp : mx;
+        has = false;
+      }
+      const uint64_t want = __builtin_amdgcn_ballot_w64(!has && more);
+      if (want) {
+        const int first = (int)__builtin_ctzll(want);
+        unsigned long long base = 0;
+        if (lane == first) base = atomicAdd(W.cursor, (unsigned long long)__builtin_popcountll(want));
+        base = ((unsigned long long)(uint32_t)__shfl((int)(uint32_t)(base >> 32), first) << 32) |
+               (uint32_t)__shfl((int)(uint32_t)base, first);
+        if (!has && more) {
+          const int64_t t = tid0 + (int64_t)base + __builtin_popcountll(want & ((1ull << lane) - 1));
+          if (t < tid1) {
+            i = order ? (int64_t)order[t] : t;
+            const float* og = R.origins + i * R.origin_stride;
+            const V3 d = normalize_dir(v3(R.dirs[3 * i], R.dirs[3 * i + 1], R.dirs[3 * i + 2]));
+            m.init(S, P, v3(og[0], og[1], og[2]), d, R.t_hit ? R.t_hit[i] : __builtin_inff(),
+                   R.visited ? R.visited + i * P.max_tiles : nullptr);
+            slot0 = i * (int64_t)cpr;
+            kr = 0;
+            run_tile = -1;
+            run_start = 0;
+            rl.reset();
+            bricks = O.bricks ? O.bricks + i * O.brick_cap : nullptr;
+            has = true;
+          } else {
+            more = false;
+          }
         }
       }
     }
     if (__builtin_amdgcn_ballot_w64(has) == 0) break;
-    if (has) {
+    full = false;
+    if (has && m.phase != FlatMarch::kDone) {
       const bool turn = tile_quorum(m.phase == FlatMarch::kTile);
       m.step(S, P, turn, bricks, O.brick_cap, on_sample);
     }
+    flush_full(stage, full, W.rec_f + slot0 + kr - 8);
   }
   const int64_t wsum = wave_sum_i64(sum);
   const int wmx = wave_max_i32(mx);

@@ -23,15 +23,33 @@
 
 namespace snisr {
 
+typedef uint32_t __attribute__((aligned(2))) u32_2;
 constexpr int kOctBlocks = 4;  // blocks per tile edge (num_block, raydiffuse_render_octree_fp16.cu:6)
 // march steps per block, taken or skipped; a block of a valid scene needs ~sqrt(3) * 16 / 0.2 < 140.
 // The cap bounds the loop for degenerate rays (zero direction: far = 1e8) and for steps below
 // zval's FP32 resolution, where zval += step would never reach far.
 constexpr int kOctMaxBlockSteps = 1 << 16;
-constexpr int kOctBatch = 2;  // samples whose loads are issued together (2: 417 us, 4: 456 us, 8: 576 us per 720p frame)
+constexpr int kOctBatch = 2;  // samples whose loads are issued together (1: 700 us, 2: 685, 3: 729 per 720p frame of 16 tiles)
 
-__device__ __forceinline__ float lerp_ab(float a, float b, float t) { return a * (1.0f - t) + b * t; }
+__device__ __forceinline__ float lerp_ab(float a, float b, float t, float u) { return a * u + b * t; }
 
+// half W of v times t, rounded once: the FP32 product of the converted half
+template <int W>
+__device__ __forceinline__ float half_times(uint32_t v, float t) {
+  float r;
+  if constexpr (W == 0)
+    asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(v), "v"(t));
+  else
+    asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(v), "v"(t));
+  return r;
+}
+
+// Bound by vector instructions (87% busy before, 46 of 64 lanes active): about 23 000 per wavefront of 64 rays, most
+// of them in the interpolation.  The halves enter it as operands of v_fma_mix_f32 (half times float, rounded once, so
+// the same bits as a conversion and a product), and the eight voxel ids of a sample are four 4-byte loads: 776 -> 658
+// us for the frame above with its rays and tile lists.  Reading a zero voxel through a selected address instead of
+// skipping empty corners' loads took 732.  Marching ahead to the next flagged sample would leave 40 of 64 steps where
+// half the cells are flagged, for about as many instructions as it saves.
 __global__ __launch_bounds__(64) void k_render_octree(snisr_octree O, const float* __restrict__ origin,
                                                       const float* __restrict__ rays_d, const int32_t* __restrict__ visited,
                                                       int64_t n, int K, int packet_w, float trans_th, float early_stop,
@@ -132,17 +150,24 @@ __global__ __launch_bounds__(64) void k_render_octree(snisr_octree O, const floa
             }
             base[b] = i0[0] * MM + i0[1] * M + i0[2];
           }
-          int16_t vid[kOctBatch][8];
+          // the two z corners of a column are neighbours in the grid: one 4-byte load per column
+          u32_2 idx[kOctBatch][4];
 #pragma unroll
           for (int b = 0; b < kOctBatch; ++b)
 #pragma unroll
-            for (int q = 0; q < 8; ++q) vid[b][q] = nodes[base[b] + (q & 1) * MM + ((q >> 1) & 1) * M + (q >> 2)];
+            for (int q = 0; q < 4; ++q)
+              idx[b][q] = *reinterpret_cast<const u32_2*>(nodes + base[b] + (q & 1) * MM + (q >> 1) * M);
           bool take[kOctBatch];
+          int vid[kOctBatch][8];
 #pragma unroll
           for (int b = 0; b < kOctBatch; ++b) {
             take[b] = live[b] && flg[b] != 0;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) vid[b][q] = take[b] ? vid[b][q] : (int16_t)-1;
+            for (int q = 0; q < 4; ++q) {
+              const int both = take[b] ? (int)idx[b][q] : -1;
+              vid[b][q] = (int)(int16_t)both;
+              vid[b][4 + q] = both >> 16;
+            }
           }
           uint2 raw[kOctBatch][8];
 #pragma unroll
@@ -159,19 +184,15 @@ __global__ __launch_bounds__(64) void k_render_octree(snisr_octree O, const floa
               inverse_near[r] = 1.0f / (zs[b] + bl);
               net_idx[r] = (int16_t)group;
             }
-            float cv[8][4];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              const _Float16* hv = reinterpret_cast<const _Float16*>(&raw[b][q]);
-#pragma unroll
-              for (int c = 0; c < 4; ++c) cv[q][c] = (float)hv[c];
-            }
+            const float tx = w[b][0], ty = w[b][1], tz = w[b][2], ux = 1.0f - tx, uy = 1.0f - ty, uz = 1.0f - tz;
             float v[4];
 #pragma unroll
             for (int ch = 0; ch < 4; ++ch) {
-              const float s0 = lerp_ab(lerp_ab(cv[0][ch], cv[1][ch], w[b][0]), lerp_ab(cv[2][ch], cv[3][ch], w[b][0]), w[b][1]);
-              const float s1 = lerp_ab(lerp_ab(cv[4][ch], cv[5][ch], w[b][0]), lerp_ab(cv[6][ch], cv[7][ch], w[b][0]), w[b][1]);
-              v[ch] = lerp_ab(s0, s1, w[b][2]);
+              const auto along_x = [&](int q) {
+                const uint32_t a = ch < 2 ? raw[b][q].x : raw[b][q].y, c = ch < 2 ? raw[b][q + 1].x : raw[b][q + 1].y;
+                return (ch & 1) ? half_times<1>(a, ux) + half_times<1>(c, tx) : half_times<0>(a, ux) + half_times<0>(c, tx);
+              };
+              v[ch] = lerp_ab(lerp_ab(along_x(0), along_x(2), ty, uy), lerp_ab(along_x(4), along_x(6), ty, uy), tz, uz);
             }
             const float interval = fminf(step, far - zs[b]);
             const float alpha = 1.0f - exp_cw(-1.0f * v[3] * interval);

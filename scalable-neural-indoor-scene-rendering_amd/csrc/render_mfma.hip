@@ -1436,24 +1436,31 @@ __global__ __launch_bounds__(512) void k_mlp_mfma(snisr_scene S, snisr_rays R, R
 }
 
 // ------------------------------------------------------------------------- ordered reduction
+// Eight lanes per ray read eight consecutive records (one 128-byte line) and every lane adds them in sample order.
+// One lane per ray read its records 16 bytes at a time, each wait exposed: 13.5 -> 5.6 us for 3001 rays, 31 -> 27
+// for 131k rays and 3.04M records.
+constexpr int kRayLanes = 8;
 __global__ __launch_bounds__(256) void k_reduce(Workspace W, int64_t n, float* __restrict__ rgb) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kRayLanes;
+  const int g = threadIdx.x % kRayLanes;
+  if (i >= n) return;  // whole groups
   const int64_t b = W.offsets[i], e = W.offsets[i + 1];
   float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
   if (e > W.cap) {
     c0 = c1 = c2 = __builtin_nanf("");
   } else {
-    for (int64_t k = b; k < e; ++k) {
-      const float4 v = W.rgbw[k];
-      c0 = c0 + v.x;
-      c1 = c1 + v.y;
-      c2 = c2 + v.z;
+    for (int64_t k = b; k < e; k += kRayLanes) {
+      float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (k + g < e) v = W.rgbw[k + g];
+#pragma unroll
+      for (int j = 0; j < kRayLanes; ++j) {
+        c0 = c0 + __shfl(v.x, j, kRayLanes);
+        c1 = c1 + __shfl(v.y, j, kRayLanes);
+        c2 = c2 + __shfl(v.z, j, kRayLanes);
+      }
     }
   }
-  rgb[3 * i] = c0;
-  rgb[3 * i + 1] = c1;
-  rgb[3 * i + 2] = c2;
+  if (g < 3) rgb[3 * i + g] = g == 0 ? c0 : (g == 1 ? c1 : c2);
 }
 
 
@@ -1492,24 +1499,42 @@ __host__ __device__ constexpr int64_t param_w_off(int in0, int wd, int L, int l)
   return s;
 }
 
-// dL/dsigma and dL/dc of every record of ray i, in reverse sample order
+// dL/dsigma and dL/dc of every record of ray i, in reverse sample order.  Eight lanes per ray take eight records from
+// the end (lane g the g-th last of them); the suffix sum is added up lane by lane in the sequential order, so the
+// results do not depend on the split.  One lane per ray moved three 16-byte pieces per record and wait: 27 -> 6.9 us
+// for 3001 rays, 230 -> 62 for 131k rays and 3.04M records (204 MB).
 __global__ __launch_bounds__(256) void k_train_comp_bwd(Workspace W, int64_t n, const float* __restrict__ g) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kRayLanes;
+  const int l = threadIdx.x % kRayLanes;
+  if (i >= n) return;  // whole groups
   const int64_t b = W.offsets[i], e = W.offsets[i + 1];
   if (e > W.cap) return;  // overflowed in the forward: no records
   const float g0 = g[3 * i], g1 = g[3 * i + 1], g2 = g[3 * i + 2];
   float suffix = 0.0f;
-  for (int64_t k = e - 1; k >= b; --k) {
-    const float4 c = W.crec[k];
-    const float4 rf = W.rec_f[k];
-    const float4 rb = W.rec_b[k];
-    const float cg = c.x * g0 + c.y * g1 + c.z * g2;
-    float ds = rb.x * (rb.y * cg - suffix);
-    suffix = suffix + rf.w * cg;
-    if (!(rb.z > 0.0f)) ds = 0.0f;
-    W.dsig[k] = ds;
-    W.rgbw[k] = make_float4(rf.w * g0, rf.w * g1, rf.w * g2, 0.0f);
+  for (int64_t k = e - 1 - l; k > b - 1 - l; k -= kRayLanes) {
+    const bool live = k >= b;
+    float4 rf = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rb = rf;
+    float cg = 0.0f;
+    if (live) {
+      const float4 c = W.crec[k];
+      rf = W.rec_f[k];
+      rb = W.rec_b[k];
+      cg = c.x * g0 + c.y * g1 + c.z * g2;
+    }
+    const float term = rf.w * cg;
+    float s = suffix;  // of the records after this lane's
+#pragma unroll
+    for (int j = 0; j < kRayLanes - 1; ++j) {
+      const float t = __shfl(term, j, kRayLanes);
+      s = l > j ? s + t : s;
+    }
+    suffix = __shfl(s + term, kRayLanes - 1, kRayLanes);
+    if (live) {
+      float ds = rb.x * (rb.y * cg - s);
+      if (!(rb.z > 0.0f)) ds = 0.0f;
+      W.dsig[k] = ds;
+      W.rgbw[k] = make_float4(rf.w * g0, rf.w * g1, rf.w * g2, 0.0f);
+    }
   }
 }
 
@@ -2187,7 +2212,7 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
 #undef SNISR_FWD
   SNISR_LAUNCHED();
   SNISR_HIP(stage_event(out, 2, st));
-  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, W, n, out->rgb);
+  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((n * kRayLanes + 255) / 256)), dim3(256), 0, st, W, n, out->rgb);
   SNISR_LAUNCHED();
   SNISR_HIP(stage_event(out, 3, st));
   return SNISR_OK;
@@ -2226,7 +2251,7 @@ int snisr_train_backward(const snisr_scene* scene, const snisr_march_params* par
   Workspace W;
   layout(n, cap, scene->n_tiles, (uint8_t*)workspace, &W,
          train_act_floats(scene->mlp_in, scene->mlp_width, scene->mlp_layers), train_frag_floats(scene));
-  hipLaunchKernelGGL(k_train_comp_bwd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, W, n, grad_rgb);
+  hipLaunchKernelGGL(k_train_comp_bwd, dim3((unsigned)((n * kRayLanes + 255) / 256)), dim3(256), 0, st, W, n, grad_rgb);
   SNISR_LAUNCHED();
   SNISR_HIP(stage_event(&ev, 1, st));
   const dim3 jgrid(train_groups(cap, scene->n_tiles, WD));

@@ -14,7 +14,7 @@
 // remainder is inf - inf).
 //
 // Against FP32 products with weights read from L2 by every wavefront (3.04M records at width 128; 530k samples
-// of the reflection MLP; us): forward 2502 -> 1146; 305 -> 108, backward 6654 -> 4344; 572 -> 314.  With
+// of the reflection MLP; us): forward 2502 -> 1146; 305 -> 108, backward 6654 -> 4240; 572 -> 301.  With
 // three BF16 parts and six products the forward took 2160; 212: under matrix load the card holds about half
 // of its nominal rate, so the products themselves are what is worth saving.
 //
@@ -318,7 +318,10 @@ __device__ __forceinline__ void quad_transpose(float (&v)[4]) {
 }
 
 // stores registers 4g .. 4g+3 (rows 8(g%4) + 4h .. +3 of feature block g / 4) of this wavefront's 32 records
-// for NG groups of a layer of width W (a multiple of 8, or 4: lane half 0 only); called by whole wavefronts
+// for NG groups of a layer of width W (a multiple of 8, or 4: lane half 0 only); called by whole wavefronts.
+// The rows are read once, by another kernel and long after: non-temporal stores keep them from displacing the weights
+// and features (backward of 3.04M records at width 128: 4420 -> 4240 us).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <int W, int NG>
 __device__ __forceinline__ void store_rows(float* __restrict__ block, const float* x, int lane) {
   const int c = lane & 31, h = lane >> 5, q = c >> 2, i = c & 3;
@@ -328,7 +331,7 @@ __device__ __forceinline__ void store_rows(float* __restrict__ block, const floa
     quad_transpose(v);
     const int b = g / 4, w = W - 32 * b < 32 ? W - 32 * b : 32;
     float* to = block + 1024 * b + 4 * (q * w + 8 * (g % 4) + 4 * h + i);
-    if (W >= 8 || h == 0) *reinterpret_cast<float4*>(to) = make_float4(v[0], v[1], v[2], v[3]);
+    if (W >= 8 || h == 0) __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(to));
   }
 }
 

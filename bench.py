@@ -117,7 +117,8 @@ def train_bench(args, dev):
     ms = (time.perf_counter() - t0) * 1e3 / args.train_steps
     n = o.shape[0]
     samples = int(ws.samples_last())
-    # forward + backward of the MLP = 3 x the forward FLOPs per sample (FP32 MFMA)
+    # forward + backward of the MLP = 3 x the forward FLOPs per sample (FP32 results; the products run as 16-bit parts,
+    # so the FP32 MFMA peak is a yardstick, not a bound)
     tflops = 3 * samples * mlp_flops_per_sample(sc.mlp_in, sc.mlp_width, sc.mlp_layers) / (ms * 1e-3) / 1e12
     return {"train_mrays_s": round(n / (ms * 1e-3) / 1e6, 3), "train_ms_per_step": round(ms, 3),
             "train_samples_per_step": samples,
@@ -630,7 +631,7 @@ def main():
     del src, dst
     extra["hbm_copy_gbs"] = round(copy_gbs, 1)
     extra["march_vs_copy_rate"] = round(march_gbs / copy_gbs, 3)
-    # plain FP32 path (one thread per ray) on the same frame, for the MFMA/FP32 speed ratio
+    # plain FP32 path (eight lanes per ray) on the same frame, for the MFMA/FP32 speed ratio
     if args.fp32_frames > 0:
         D.render_fp32(ds, origin, rays_d, t_hit=t_hit, image_width=W)
         torch.cuda.synchronize()

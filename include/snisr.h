@@ -134,7 +134,7 @@ int snisr_compute_rays(const float* intrinsic, const float* c2w, int32_t H, int3
 int snisr_trace_tiles(const snisr_scene* scene, const float* origin, const float* rays_d, int64_t n, int32_t K,
                       int32_t* visited, void* stream);
 
-/* A3+A4+A5+A7 — one-thread-per-ray FP32 render: tile DDA, brick DDA, uniform march,
+/* A3+A4+A5+A7 — FP32 render, eight lanes per ray: tile DDA, brick DDA, uniform march,
  * trilinear sigma + features, per-tile FP32 MLP, early-terminating compositing.  Replaces
  * rendering_diffuse_octree_fp16 (rendering/src/raydiffuse_render_octree_fp16.cu:238-287,
  * include/raydiffuse_render_octree.h:7-21) and the FP32 marcher render_diffuse_kernel

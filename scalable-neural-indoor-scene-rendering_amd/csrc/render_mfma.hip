@@ -1466,7 +1466,7 @@ __global__ __launch_bounds__(256) void k_reduce(Workspace W, int64_t n, float* _
 
 // ------------------------------------------------------------------------- training (FP32)
 // Forward: same count/scan/emit (+ interval, T after, sigma per record) and tile sort as the render,
-// then the per-record FP32 MLP on FP32 MFMA (k_train_mma).  Backward: a per-ray reverse pass gives
+// then the per-record MLP as split 16-bit MFMA products (k_train_mma).  Backward: a per-ray reverse pass gives
 // dL/dc and dL/dsigma of every record; k_train_mma recomputes the MLP forward of every record
 // (segment recomputation), writes each layer's input rows and output-delta rows, backpropagates to
 // the features and scatter-adds the trilinear adjoint into the feature and density gradients; a
@@ -2198,7 +2198,7 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   hipLaunchKernelGGL(k_tile_scatter, dim3(kSortGrid), dim3(kSortBlock), 0, st, W);
   SNISR_LAUNCHED();
   SNISR_HIP(stage_event(out, 1, st));
-  {  // this step's weights as FP32 MFMA fragments (the backward reads the same copy)
+  {  // this step's weights as two-part FP16 fragments (the backward reads the same copy)
     hipLaunchKernelGGL(k_pack_train, dim3((unsigned)(scene->n_tiles * L)), dim3(kPackThreads), 0, st, scene->mlp_params,
                        scene->mlp_stride, W.frag, scene->mlp_in, WD, L);
     SNISR_LAUNCHED();

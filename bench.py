@@ -117,8 +117,8 @@ def train_bench(args, dev):
     ms = (time.perf_counter() - t0) * 1e3 / args.train_steps
     n = o.shape[0]
     samples = int(ws.samples_last())
-    # forward + backward of the MLP = 3 x the forward FLOPs per sample (FP32 results; the products run as 16-bit parts,
-    # so the FP32 MFMA peak is a yardstick, not a bound)
+    # forward + backward of the MLP = 3 x the forward FLOPs per sample (the layer products on FP32 MFMA; the weight
+    # gradients run as six BF16 products, so the FP32 MFMA peak is a yardstick for them, not a bound)
     tflops = 3 * samples * mlp_flops_per_sample(sc.mlp_in, sc.mlp_width, sc.mlp_layers) / (ms * 1e-3) / 1e12
     return {"train_mrays_s": round(n / (ms * 1e-3) / 1e6, 3), "train_ms_per_step": round(ms, 3),
             "train_samples_per_step": samples,

@@ -7,11 +7,11 @@
 // outputs, LeakyReLU 0.01) of the reference's training configuration (training/config/cfg.yaml:38-46),
 // used for the compute_voxels bake, the background samples and the specular branch.
 //
-// The products run on FP16 MFMA with every FP32 operand as two parts (train_mma.hpp): a wavefront takes 32
-// samples as the 32 columns, each half of a sample's two lanes computes half of its positional encoding
-// (15 sin/cos pairs), and every layer's output (the D layout) is the next layer's B operand, so activations never leave registers; the four wavefronts of a workgroup share
-// the weights, packed once per call as forward and transposed fragments, through LDS.  The forward writes
-// only the outputs.  The backward recomputes the forward from the points, keeps the activation signs as bit
+// The products run on FP32 MFMA (train_mma.hpp): a wavefront takes 32 samples as the 32 columns, each half of a
+// sample's two lanes computes half of its positional encoding (15 sin/cos pairs), and every layer's output
+// (the D layout) is the next layer's B operand, so activations never leave registers; the four wavefronts of a
+// workgroup share the weights, packed once per call as forward and transposed fragments, through LDS.  The
+// forward writes only the outputs.  The backward recomputes the forward from the points, keeps the activation signs as bit
 // masks, writes each layer's input row and output-delta row, and a second kernel reduces the weight
 // gradients dW = sum delta (x) input from the rows.
 #include "snisr_common.hpp"
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
                                                       float* __restrict__ out, const float* __restrict__ g_out,
                                                       float* __restrict__ rows) {
   static_assert(NOUT % 4 == 0 && NOUT <= 32, "output rows in whole 4-row groups of one block");
-  constexpr int NKO = (NOUT + 15) / 16;   // k-chunks of the output layer's transposed product
+  constexpr int NSO = NOUT <= 8 ? 4 : 16;  // steps of the output layer's transposed product
   constexpr int NOP = NOUT <= 4 ? 4 : 32;  // delta pitch of the output layer
   __shared__ __align__(16) uint8_t w_lds[2 * kChunkBytes];
   const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
@@ -156,8 +156,7 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
   const float* bias = P + bias_off;
   float a[32];
   uint64_t mask[8];
-  const float* winv = P + bias_off + 64 * (depth - 1) + 32;
-  stream_layer<kPNs0 / 8, 2>(fs, x0, lane, winv[0], bias, [&](int r, float v) { a[r] = v > 0.0f ? v : slope * v; });
+  stream_layer<kPNs0, 2>(fs, x0, lane, bias, [&](int r, float v) { a[r] = v > 0.0f ? v : slope * v; });
   uint64_t mk_last = 0;  // mask of the output layer's input
 #pragma unroll
   for (int l = 1; l < 8; ++l) {
@@ -171,7 +170,7 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
       break;
     }
     float y[32];
-    stream_layer<4, 2>(fs, a, lane, winv[l], bias, [&](int r, float v) { y[r] = v > 0.0f ? v : slope * v; });
+    stream_layer<32, 2>(fs, a, lane, bias, [&](int r, float v) { y[r] = v > 0.0f ? v : slope * v; });
 #pragma unroll
     for (int r = 0; r < 32; ++r) a[r] = y[r];
   }
@@ -180,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
     fs.step();
   } else {
     float z[16];
-    stream_layer<4, 1>(fs, a, lane, winv[depth - 1], bias, [&](int r, float v) { z[r] = v; });
+    stream_layer<32, 1>(fs, a, lane, bias, [&](int r, float v) { z[r] = v; });
     if (valid) {
 #pragma unroll
       for (int g = 0; g < 4; ++g)
@@ -190,9 +189,9 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
   }
   // ---- backward: output delta (register s: row tr_row(s, h)), then d_{l-1} = (W_l^T d_l) * leaky'
   const int64_t d_base = (int64_t)depth * in_rows;  // delta rows follow the input rows
-  float dout[8 * NKO];
+  float dout[NSO];
 #pragma unroll
-  for (int g = 0; g < 2 * NKO; ++g) {
+  for (int g = 0; g < NSO / 4; ++g) {
     float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (valid && 8 * g + 4 * h < NOUT) v = *reinterpret_cast<const float4*>(g_out + j * NOUT + 8 * g + 4 * h);
     dout[4 * g] = v.x;
@@ -202,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
   }
   if (any) store_rows<NOP, NOP <= 4 ? 1 : 4>(rows + d_base + (int64_t)(depth - 1) * in_rows + blk * NOP, dout, lane);
   float d[32];
-  stream_layer<NKO, 2>(fs, dout, lane, winv[depth - 1], nullptr,
+  stream_layer<NSO, 2>(fs, dout, lane, nullptr,
                        [&](int r, float v) { d[r] = leaky_mask(mk_last, r, v, slope); });
 #pragma unroll
   for (int l = 6; l >= 0; --l) {
@@ -211,7 +210,7 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
     if (any) store_rows<kPW, 8>(rows + d_base + (int64_t)l * in_rows + blk * kPW, d, lane);
     if (l == 0) break;
     float e[32];
-    stream_layer<4, 2>(fs, d, lane, winv[l], nullptr, [&](int r, float v) { e[r] = leaky_mask(mask[l], r, v, slope); });
+    stream_layer<32, 2>(fs, d, lane, nullptr, [&](int r, float v) { e[r] = leaky_mask(mask[l], r, v, slope); });
 #pragma unroll
     for (int r = 0; r < 32; ++r) d[r] = e[r];
   }

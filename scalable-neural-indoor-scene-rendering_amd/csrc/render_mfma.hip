@@ -1466,7 +1466,7 @@ __global__ __launch_bounds__(256) void k_reduce(Workspace W, int64_t n, float* _
 
 // ------------------------------------------------------------------------- training (FP32)
 // Forward: same count/scan/emit (+ interval, T after, sigma per record) and tile sort as the render,
-// then the per-record MLP as split 16-bit MFMA products (k_train_mma).  Backward: a per-ray reverse pass gives
+// then the per-record FP32 MLP on FP32 MFMA (k_train_mma).  Backward: a per-ray reverse pass gives
 // dL/dc and dL/dsigma of every record; k_train_mma recomputes the MLP forward of every record
 // (segment recomputation), writes each layer's input rows and output-delta rows, backpropagates to
 // the features and scatter-adds the trilinear adjoint into the feature and density gradients; a
@@ -1560,7 +1560,7 @@ __global__ __launch_bounds__(256, 2) void k_train_dw(Workspace W, int64_t mlp_st
   else dw_layer<WD, WD, WD, WD>(D, A, b0, b1, G, red, [](int i) { return i; });
 }
 
-// The training MLP's matrix helpers (operand split, fragment layout, packing, staging) are in train_mma.hpp.
+// The training MLP's matrix helpers (fragment layout, packing, staging) are in train_mma.hpp.
 
 __global__ __launch_bounds__(kPackThreads) void k_pack_train(const float* __restrict__ src, int64_t src_stride,
                                                              float* __restrict__ dst, int in0, int wd, int L) {
@@ -1572,7 +1572,7 @@ __global__ __launch_bounds__(kPackThreads) void k_pack_train(const float* __rest
 template <int F, int WD, int L, bool HALF, bool BWD>
 __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays R, Workspace W, float* __restrict__ dsigma,
                                                    float* __restrict__ dfeats) {
-  constexpr int IN = F + 15, NS0 = tr_ns0(IN), NB = WD / 32, NKH = WD / 16;
+  constexpr int IN = F + 15, NS0 = tr_ns0(IN), NB = WD / 32, NSH = WD / 2;
   static_assert(F % 8 == 0 && F <= 32, "feature rows must fill whole 8-row groups of the first block");
   static_assert(WD % 32 == 0 && WD <= 128 && L >= 2 && L <= 8, "MLP shape (one 64-bit ReLU mask per layer)");
   static_assert(NS0 % 8 == 0 && in_pad_of(IN, WD, 0) == 2 * NS0, "whole k-chunks of inputs");
@@ -1640,7 +1640,6 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
     x0[4 * g + 3] = e.w;
   }
   const float* bias = W.frag + (int64_t)tile * STRIDE + tr_bias_off(IN, WD, L, 0, 3);
-  const float* winv = W.frag + (int64_t)tile * STRIDE + tr_scale_off(IN, WD, L, 3);
   float* act = W.act;
   // rows of this wavefront's 32-record block, as the weight-gradient reduction reads them (padding records
   // have zero deltas)
@@ -1649,7 +1648,7 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
   float a[NB * 16];
   uint64_t mask[L];
   auto relu = [&](int r, float v) { a[r] = v > 0.0f ? v : 0.0f; };
-  stream_layer<NS0 / 8, NB>(fs, x0, lane, winv[0], bias, relu);
+  stream_layer<NS0, NB>(fs, x0, lane, bias, relu);
 #pragma unroll
   for (int l = 1; l < L; ++l) {
     bias += 32 * NB;
@@ -1659,7 +1658,7 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
     if (BWD && any) store_rows<WD, NB * 4>(act + NJ * act_a_off(IN, WD, L, l) + (j - col) * WD, a, lane);
     if (l < L - 1) {
       float y[NB * 16];
-      stream_layer<NKH, NB>(fs, a, lane, winv[l], bias, [&](int r, float v) { y[r] = v > 0.0f ? v : 0.0f; });
+      stream_layer<NSH, NB>(fs, a, lane, bias, [&](int r, float v) { y[r] = v > 0.0f ? v : 0.0f; });
 #pragma unroll
       for (int r = 0; r < NB * 16; ++r) a[r] = y[r];
     }
@@ -1667,7 +1666,7 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
   load_record();  // of the next group
   // ---- output layer: rows 0..2 (lane half 0, registers 0..2)
   float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
-  stream_layer<NKH, 1>(fs, a, lane, winv[L - 1], bias, [&](int r, float v) {
+  stream_layer<NSH, 1>(fs, a, lane, bias, [&](int r, float v) {
     if (r == 0) c0 = sigmoid_cw(v);
     if (r == 1) c1 = sigmoid_cw(v);
     if (r == 2) c2 = sigmoid_cw(v);
@@ -1681,7 +1680,7 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
     continue;
   }
   // ---- output delta from dL/dc (written into rgbw by the compositing adjoint)
-  float dout[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  float dout[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   if (valid && h == 0) {
     const float4 dc = W.rgbw[kc];
     dout[0] = dc.x * c0 * (1.0f - c0);
@@ -1691,14 +1690,14 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
   if (any) store_rows<4, 1>(act + NJ * act_d_off(IN, WD, L, L - 1) + (j - col) * 4, dout, lane);
   // ---- backpropagate: d_{l-1} = mask_l (W_l^T d_l)
   float d[NB * 16];
-  stream_layer<1, NB>(fs, dout, lane, winv[L - 1], nullptr,
+  stream_layer<4, NB>(fs, dout, lane, nullptr,
                       [&](int r, float v) { d[r] = ((mask[L - 1] >> (r & 63)) & 1) ? v : 0.0f; });
 #pragma unroll
   for (int l = L - 2; l >= 0; --l) {
     if (any) store_rows<WD, NB * 4>(act + NJ * act_d_off(IN, WD, L, l) + (j - col) * WD, d, lane);
     if (l > 0) {
       float e[NB * 16];
-      stream_layer<NKH, NB>(fs, d, lane, winv[l], nullptr,
+      stream_layer<NSH, NB>(fs, d, lane, nullptr,
                             [&](int r, float v) { e[r] = ((mask[l] >> (r & 63)) & 1) ? v : 0.0f; });
 #pragma unroll
       for (int r = 0; r < NB * 16; ++r) d[r] = e[r];
@@ -1706,7 +1705,7 @@ __global__ __launch_bounds__(256, 2) void k_train_mma(snisr_scene S, snisr_rays 
   }
   // ---- dL/d(features): rows 0..F-1 of W_0^T d_0
   float df[16];
-  stream_layer<NKH, 1>(fs, d, lane, winv[0], nullptr, [&](int r, float v) { df[r] = v; });
+  stream_layer<NSH, 1>(fs, d, lane, nullptr, [&](int r, float v) { df[r] = v; });
   __syncthreads();  // the weight stream's buffers become the exchange area
   // ---- trilinear adjoint.  The wave's 32 records go through LDS so that each atomic instruction
   // covers whole feature rows (64 / F records x F contiguous features) instead of 64 scattered
@@ -2198,7 +2197,7 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   hipLaunchKernelGGL(k_tile_scatter, dim3(kSortGrid), dim3(kSortBlock), 0, st, W);
   SNISR_LAUNCHED();
   SNISR_HIP(stage_event(out, 1, st));
-  {  // this step's weights as two-part FP16 fragments (the backward reads the same copy)
+  {  // this step's weights as MFMA fragments (the backward reads the same copy)
     hipLaunchKernelGGL(k_pack_train, dim3((unsigned)(scene->n_tiles * L)), dim3(kPackThreads), 0, st, scene->mlp_params,
                        scene->mlp_stride, W.frag, scene->mlp_in, WD, L);
     SNISR_LAUNCHED();

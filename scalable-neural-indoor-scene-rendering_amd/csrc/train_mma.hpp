@@ -1,26 +1,18 @@
 // Matrix-product building blocks of the FP32 training MLPs (the feature-scene training chain and the
-// positional-encoding MLP): FP32 operands as sums of 16-bit parts, the packing of the weights, their staging
-// through LDS and the product of one layer.
+// positional-encoding MLP): the packing of the weights, their staging through LDS and the product of one
+// layer on v_mfma_f32_32x32x2_f32, and the splitting of the weight gradients' operands.
 //
-// A layer's product W x runs on v_mfma_f32_32x32x16_f16 with both operands as two FP16 parts: the operand is
-// scaled by a power of two so that its largest magnitude (of the layer's weights; of the activation column)
-// lies in [2^14, 2^15), hi = the scaled value rounded to FP16, lo = the rounded remainder, and
-// W x = hi hi + hi lo + lo hi, accumulated in FP32 and scaled back exactly.  hi + lo keeps 22 bits and lo lo
-// is below 2^-22, both of random sign; a value 2^-16 of its column's largest still keeps them.  The three
-// products sum 16 terms per rounding where v_mfma_f32_32x32x2_f32 sums two, and the errors against 64 bits
-// are those of the FP32 products or smaller (relative, FP32 products | these: parameter gradients of the
-// 530k-sample reflection step 9.0e-6 | 4.7e-6, of the diffuse step 3.1e-5 | 3.1e-5, feature gradients of the
-// 131k-ray step 9.1e-3 | 9.1e-3, where the march's positions set them).  An infinite operand gives NaN (its
-// remainder is inf - inf).
+// The layer products take FP32 operands as they are and add them in one order (the bias, then the inputs in
+// step order), so a value, an infinity and the sign of a hidden value near zero, which decides its ReLU, are
+// what an FP32 chain gives.  Two-part FP16 operands with a power-of-two scale per layer were built and taken
+// back, though they were faster (3.04M records at width 128: forward 1.15 ms against 2.45, backward 4.24
+// against 5.90): they keep 22 bits, units far below their layer's largest weight lost bits and in the end
+// vanished, an infinity became NaN and then 0 in the ReLU, and the other rounding of hidden values near zero
+// moved the parameter gradients of the 530k-sample reflection step by 4e-5.
 //
-// Against FP32 products with weights read from L2 by every wavefront (3.04M records at width 128; 530k samples
-// of the reflection MLP; us): forward 2502 -> 1146; 305 -> 108, backward 6654 -> 4240; 572 -> 301.  With
-// three BF16 parts and six products the forward took 2160; 212: under matrix load the card holds about half
-// of its nominal rate, so the products themselves are what is worth saving.
-//
-// Sums over records (the weight gradients) have no common scale: their operands are split into three BF16
-// parts, which keep the range and all 24 bits of FP32, and multiplied as six products (what is left out is
-// below 2^-26).
+// Sums over records (the weight gradients) decide no sign: their operands are split into three BF16 parts,
+// which keep the range and all 24 bits of FP32, and multiplied as six products (what is left out is below
+// 2^-25).  An infinite operand, or one above the largest BF16 number (3.39e38), makes its row NaN.
 #pragma once
 
 #include "mfma_ops.hpp"
@@ -29,23 +21,23 @@
 namespace snisr {
 
 // One wavefront takes 32 records of one tile as the 32 columns, so every layer is W (out x in) times a
-// 32-column block of activations.  Lane layouts of v_mfma_f32_32x32x16 (h = lane / 32, c = lane % 32):
-//   A:  lane holds A[row c][k slots 8h .. 8h+7]      B:  lane holds B[k slots 8h .. 8h+7][column c]
+// 32-column block of activations.  Lane layouts of v_mfma_f32_32x32x2_f32 (h = lane / 32, c = lane % 32):
+//   A:  lane holds A[row c][k = h]        B:  lane holds B[k = h][column c]
 //   D:  lane holds rows 8(r/4) + 4h + (r%4), r = 0..15, of column c
 // Register s of a lane's activations holds row tr_row(s, h): the order in which the D blocks of a layer
-// come out.  K slot e of half h in k-chunk kc is row tr_row(8 kc + e, h), so the B operand of a chunk is
-// registers 8 kc .. 8 kc + 7 of the previous layer's output and activations never leave registers.
-// Layer 0's inputs (features, then the view encoding) follow the same row order.
+// come out.  Step s of a product pairs the rows tr_row(s, 0) and tr_row(s, 1), so its B operand is register s
+// of the previous layer's output and activations never leave registers.  Layer 0's inputs (features, then
+// the view encoding) follow the same row order.
 __host__ __device__ constexpr int tr_row(int s, int h) { return 32 * (s / 16) + 8 * ((s % 16) / 4) + 4 * h + (s % 4); }
 // registers of layer 0's inputs: whole 8-row groups
 __host__ __device__ constexpr int tr_ns0(int in0) { return 16 * (in0 / 32) + 4 * ((in0 % 32 + 7) / 8); }
 
-// Packed weights: a fragment is 32 output rows x 16 k, its two parts of 64 lanes x 16 bytes; the fragments
-// of a layer are ordered k-chunk by k-chunk, output block by output block, and padded to whole groups of
-// kChunkFrags, the unit that is staged through LDS.  Order: the forward layers 0 .. L-1, the transposed
-// layers L-1 .. 0, i.e. the order in which the kernels read them; then the biases (32 floats per output
-// block, in the D layout) and one factor per layer, the inverse of its weights' scale.
-constexpr int kPartBytes = 1024, kFragBytes = 2 * kPartBytes, kChunkFrags = 8, kChunkBytes = kChunkFrags * kFragBytes;
+// Packed weights: a fragment is 32 output rows x 8 steps (16 inputs), as two pieces of 64 lanes x 4 steps; the
+// fragments of a layer are ordered k-chunk by k-chunk, output block by output block, and padded to whole
+// groups of kChunkFrags, the unit that is staged through LDS.  Order: the forward layers 0 .. L-1, the
+// transposed layers L-1 .. 0, i.e. the order in which the kernels read them; then the biases (32 floats per
+// output block, in the D layout).
+constexpr int kPieceBytes = 1024, kFragBytes = 2 * kPieceBytes, kChunkFrags = 8, kChunkBytes = kChunkFrags * kFragBytes;
 __host__ __device__ constexpr int tr_nob(int wd, int L, int l) { return l == L - 1 ? 1 : wd / 32; }
 __host__ __device__ constexpr int tr_nkf(int in0, int wd, int l) { return l == 0 ? (tr_ns0(in0) + 7) / 8 : wd / 16; }
 __host__ __device__ constexpr int tr_nib(int wd, int l) { return l == 0 ? 1 : wd / 32; }
@@ -63,40 +55,15 @@ __host__ __device__ constexpr int tr_bwd_chunk(int in0, int wd, int L, int l, in
   for (int m = L - 1; m > l; --m) n += tr_chunks(tr_nkb(wd, L, m, nout) * tr_nib(wd, m));
   return n;
 }
-// float offset of layer l's biases in the packed block, and the block's floats
+// float offset of layer l's biases in the packed block
 __host__ __device__ constexpr int64_t tr_bias_off(int in0, int wd, int L, int l, int nout) {
   int64_t o = (int64_t)tr_bwd_chunk(in0, wd, L, -1, nout) * (kChunkBytes / 4);
   for (int m = 0; m < l; ++m) o += 32 * tr_nob(wd, L, m);
   return o;
 }
-// float offset of the layers' factors, and the floats of a packed block
-__host__ __device__ constexpr int64_t tr_scale_off(int in0, int wd, int L, int nout) { return tr_bias_off(in0, wd, L, L, nout); }
+// floats of a packed block
 __host__ __device__ constexpr int64_t tr_stride(int in0, int wd, int L, int nout) {
-  return (tr_scale_off(in0, wd, L, nout) + L + 63) / 64 * 64;
-}
-
-// power of two that brings a largest magnitude into [2^14, 2^15), and its inverse (magnitudes below 2^-112
-// count as 2^-112)
-__device__ __forceinline__ void range_scale(float largest, float& scale, float& inverse) {
-  uint32_t e = __float_as_uint(largest) >> 23;
-  e = e < 15u ? 15u : (e > 254u ? 254u : e);
-  scale = __uint_as_float((268u - e) << 23);
-  inverse = __uint_as_float((e - 14u) << 23);
-}
-
-// hi + lo of eight scaled values
-struct Pair8 {
-  f16x8 hi, lo;
-};
-__device__ __forceinline__ Pair8 pair8(const float* v, float scale) {
-  Pair8 s;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const _Float16 h = (_Float16)(v[e] * scale);
-    s.hi[e] = h;
-    s.lo[e] = (_Float16)__builtin_fmaf(v[e], scale, -(float)h);
-  }
-  return s;
+  return (tr_bias_off(in0, wd, L, L, nout) + 63) / 64 * 64;
 }
 
 // x = hi + mid + lo of eight values, each part rounded to nearest BF16
@@ -141,25 +108,14 @@ __device__ __forceinline__ void mma_split(const Split8 (&a)[NA], const Split8 (&
 
 namespace {
 constexpr int kPackThreads = 512;
-// One workgroup per layer and tile: the largest magnitude of the layer's weights, then its forward and
-// transposed fragments, its biases and its factor (mlp_params layout: per layer W[out][in], then b[out]; the
-// last layer has nout <= 32 rows).  in_of(row): the input at row `row` of layer 0's products.
+// One workgroup per layer and tile: the layer's forward and transposed fragments and its biases (mlp_params
+// layout: per layer W[out][in], then b[out]; the last layer has nout <= 32 rows).  in_of(row): the input at
+// row `row` of layer 0's products.
 template <class InOf>
 __device__ __forceinline__ void pack_train_layer(const float* __restrict__ P, float* __restrict__ block, int in0, int wd,
                                                  int L, int l, int nout, InOf in_of) {
-  __shared__ float wmax[kPackThreads / 64];
   for (int m = 0; m < l; ++m) P += (int64_t)((m == 0 ? in0 : wd) + 1) * wd;
   const int in = l == 0 ? in0 : wd, out = l == L - 1 ? nout : wd;
-  float mx = 0.0f;
-  for (int q = threadIdx.x; q < in * out; q += kPackThreads) mx = fmaxf(mx, fabsf(P[q]));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  for (int w = 0; w < kPackThreads / 64; ++w) mx = fmaxf(mx, wmax[w]);
-  float scale, inverse;
-  range_scale(mx, scale, inverse);
-  if (threadIdx.x == 0) block[tr_scale_off(in0, wd, L, nout) + l] = inverse;
   const int nob = tr_nob(wd, L, l);
   float* bias = block + tr_bias_off(in0, wd, L, l, nout);
   for (int q = threadIdx.x; q < 32 * nob; q += kPackThreads) {
@@ -181,9 +137,10 @@ __device__ __forceinline__ void pack_train_layer(const float* __restrict__ P, fl
         if (l == 0) i = in_of(i);
         v[e] = kc < nk && o < out && i < in ? P[(int64_t)o * in + i] : 0.0f;
       }
-      const Pair8 s = pair8(v, scale);
-      *reinterpret_cast<f16x8*>(to + (int64_t)f * kFragBytes + lane * 16) = s.hi;
-      *reinterpret_cast<f16x8*>(to + (int64_t)f * kFragBytes + kPartBytes + lane * 16) = s.lo;
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        *reinterpret_cast<float4*>(to + (int64_t)f * kFragBytes + p * kPieceBytes + lane * 16) =
+            make_float4(v[4 * p], v[4 * p + 1], v[4 * p + 2], v[4 * p + 3]);
     }
   }
 }
@@ -191,7 +148,7 @@ __device__ __forceinline__ void pack_train_layer(const float* __restrict__ P, fl
 
 // The weight stream of a 256-thread workgroup: chunks of kChunkFrags fragments go from global memory
 // through registers into one of two LDS buffers, the next chunk's loads in flight while the current one is
-// used.  Without the staging every wavefront would read every fragment from L2 (3 KB per six products).
+// used.  Without the staging every wavefront would read every fragment from L2 (2 KB per eight products).
 // All wavefronts of the workgroup call start() and the same number of step()s.
 struct FragStream {
   static constexpr int kThreads = 256;
@@ -233,60 +190,42 @@ struct FragStream {
   }
 };
 
-// largest magnitude of this lane's column: N values here, the others in the lane of the other half
-template <int N>
-__device__ __forceinline__ float column_max(const float* x) {
-  float m = 0.0f;
-#pragma unroll
-  for (int r = 0; r < N; ++r) m = fmaxf(m, fabsf(x[r]));
-  float lo, hi;
-  swap_halves(m, lo, hi);
-  return fmaxf(lo, hi);
-}
-
-// out(i, y) for register i of the NOB output blocks, y = (the layer's fragments times x) + bias; x: registers
-// s (row tr_row(s, h)) over NK k-chunks, at least 8 NK values; weight_inv: the layer's factor; bias: NOB
-// blocks of 32 floats, or NULL.  All output blocks advance together, so x is split once and consecutive
-// products are independent; the small products come first in a k-chunk.
-template <int NK, int NOB, class Out>
-__device__ __forceinline__ void stream_layer(FragStream& fs, const float* x, int lane, float weight_inv,
-                                             const float* __restrict__ bias, Out out) {
-  static_assert(kChunkFrags % NOB == 0, "whole k-chunks per staged chunk");
-  constexpr int KPC = kChunkFrags / NOB;
-  float scale, inv;
-  range_scale(column_max<8 * NK>(x), scale, inv);
-  inv *= weight_inv;
+// out(i, y) for register i of the NOB output blocks, y = bias + the layer's fragments times x, added in step
+// order; x: registers s (row tr_row(s, h)) over NS steps; bias: NOB blocks of 32 floats, or NULL for zeros.  All
+// output blocks advance together, so consecutive products are independent.
+template <int NS, int NOB, class Out>
+__device__ __forceinline__ void stream_layer(FragStream& fs, const float* x, int lane, const float* __restrict__ bias,
+                                             Out out) {
+  static_assert(kChunkFrags % NOB == 0 && NS % 4 == 0, "whole k-chunks per staged chunk, whole pieces");
+  constexpr int KPC = kChunkFrags / NOB, NK = (NS + 7) / 8;
   f32x16 acc[NOB];
 #pragma unroll
-  for (int ob = 0; ob < NOB; ++ob) acc[ob] = f32x16{};
+  for (int ob = 0; ob < NOB; ++ob) acc[ob] = bias ? bias_block(bias, ob, lane >> 5) : f32x16{};
 #pragma unroll
   for (int k0 = 0; k0 < NK; k0 += KPC) {
-    const uint8_t* A = fs.step();
+    const uint8_t* A = fs.step() + lane * 16;
 #pragma unroll
-    for (int k = 0; k < KPC; ++k)
-      if (k0 + k < NK) {
-        f16x8 hi[NOB], lo[NOB];
-        const Pair8 b = pair8(x + 8 * (k0 + k), scale);
+    for (int q = 0; q < 2 * KPC; ++q) {
+      const int s = 8 * k0 + 4 * q;  // first of the four steps of piece q % 2 of k-chunk k0 + q / 2
+      if (s >= NS) break;
+      float4 a[NOB];
 #pragma unroll
-        for (int ob = 0; ob < NOB; ++ob) {
-          hi[ob] = load_frag<f16x8>(A + (k * NOB + ob) * kFragBytes + lane * 16);
-          lo[ob] = load_frag<f16x8>(A + (k * NOB + ob) * kFragBytes + kPartBytes + lane * 16);
-        }
+      for (int ob = 0; ob < NOB; ++ob)
+        a[ob] = *reinterpret_cast<const float4*>(A + (q / 2 * NOB + ob) * kFragBytes + q % 2 * kPieceBytes);
 #pragma unroll
-        for (int ob = 0; ob < NOB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[ob], b.hi, acc[ob], 0, 0, 0);
+      for (int ob = 0; ob < NOB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[ob].x, x[s], acc[ob], 0, 0, 0);
 #pragma unroll
-        for (int ob = 0; ob < NOB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[ob], b.lo, acc[ob], 0, 0, 0);
+      for (int ob = 0; ob < NOB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[ob].y, x[s + 1], acc[ob], 0, 0, 0);
 #pragma unroll
-        for (int ob = 0; ob < NOB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[ob], b.hi, acc[ob], 0, 0, 0);
-      }
+      for (int ob = 0; ob < NOB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[ob].z, x[s + 2], acc[ob], 0, 0, 0);
+#pragma unroll
+      for (int ob = 0; ob < NOB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[ob].w, x[s + 3], acc[ob], 0, 0, 0);
+    }
   }
 #pragma unroll
-  for (int ob = 0; ob < NOB; ++ob) {
-    f32x16 b = f32x16{};
-    if (bias) b = bias_block(bias, ob, lane >> 5);
+  for (int ob = 0; ob < NOB; ++ob)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) out(16 * ob + r, bias ? __builtin_fmaf(acc[ob][r], inv, b[r]) : acc[ob][r] * inv);
-  }
+    for (int r = 0; r < 16; ++r) out(16 * ob + r, acc[ob][r]);
 }
 
 __device__ __forceinline__ void store4(float* p, const float* v) {

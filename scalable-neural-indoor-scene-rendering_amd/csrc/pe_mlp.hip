@@ -7,11 +7,11 @@
 // outputs, LeakyReLU 0.01) of the reference's training configuration (training/config/cfg.yaml:38-46),
 // used for the compute_voxels bake, the background samples and the specular branch.
 //
-// The products run on FP32 MFMA (train_mma.hpp): a wavefront takes 32 samples as the 32 columns, each half of a
-// sample's two lanes computes half of its positional encoding (15 sin/cos pairs), and every layer's output
-// (the D layout) is the next layer's B operand, so activations never leave registers; the four wavefronts of a
-// workgroup share the weights, packed once per call as forward and transposed fragments, through LDS.  The
-// forward writes only the outputs.  The backward recomputes the forward from the points, keeps the activation signs as bit
+// The products run on FP32 MFMA (train_mma.hpp): a wavefront takes 32 samples as the 32 columns, computes
+// their positional encoding cooperatively (30 sin/cos pairs per sample spread over the lanes, through LDS), and
+// every layer's output (the D layout) is the next layer's B operand, so activations never leave registers; the
+// four wavefronts of a workgroup share the weights, packed once per call as forward and transposed fragments,
+// through LDS.  The forward writes only the outputs.  The backward recomputes the forward from the points, keeps the activation signs as bit
 // masks, writes each layer's input row and output-delta row, and a second kernel reduces the weight
 // gradients dW = sum delta (x) input from the rows.
 #include "snisr_common.hpp"
@@ -55,53 +55,8 @@ __host__ __device__ inline int64_t pe_d_off(int l, int L, int depth, int n_out, 
 }
 
 constexpr int kPIn = 63;                 // encoding width (3 + 6 L)
-constexpr int kPNs0 = tr_ns0(kPIn);      // input registers of layer 0 (rows 0..63)
-
-// The encoding's inputs in layer 0's row order: lane half h holds the bands 5h .. 5h+4, so that no value
-// crosses lanes.  Register s of half h: s = 0: x or z; s = 1: y or nothing; then band by band sin x, sin y,
-// sin z, cos x, cos y, cos z.  pe_input(row) is the input at a row (63: none), row = tr_row(s, h).
-__host__ __device__ constexpr int pe_input(int row) {
-  const int h = (row / 4) % 2, s = 16 * (row / 32) + 4 * (row % 32 / 8) + row % 4;
-  if (s < 2) return h == 0 ? s : (s == 0 ? 2 : 63);
-  return 3 + 30 * h + s - 2;
-}
-
-// sin and cos of 2^f v for f = 5h .. 5h+4, h = lane half.  v / (2 pi) is formed once as hi + lo; scaling it by
-// 2^f is exact, and so is taking off the nearest quarter turn, so every band starts from an angle within
-// pi / 4 that carries the rounding of that quotient's 48 bits only; Taylor's series to the 9th and 10th
-// power are then below half an ulp.  Above 2^12 (a band then passes 2^21 turns) the library function takes
-// over for the whole wavefront.
-__device__ __forceinline__ void pe_bands(float v, int h, float (&sn)[5], float (&cs)[5]) {
-  constexpr float k1 = 0.15915494309189535f;                        // 1 / (2 pi) rounded
-  constexpr float k2 = (float)(0.15915494309189533577 - (double)k1);
-  constexpr float turn = 6.283185307179586f;
-  float f = h ? 32.0f : 1.0f;
-  if (__builtin_amdgcn_ballot_w64(!(fabsf(v) < 4096.0f))) {
-#pragma unroll
-    for (int q = 0; q < 5; ++q, f *= 2.0f) sincosf(f * v, &sn[q], &cs[q]);
-    return;
-  }
-  const float hi = v * k1, lo = __builtin_fmaf(v, k2, __builtin_fmaf(v, k1, -hi));
-#pragma unroll
-  for (int q = 0; q < 5; ++q, f *= 2.0f) {
-    const float a = f * hi, n = __builtin_rintf(4.0f * a);
-    const float u = __builtin_fmaf(f, lo, __builtin_fmaf(-0.25f, n, a)) * turn, u2 = u * u;
-    float s = 2.7557319e-6f, c = -2.7557319e-7f;
-    s = __builtin_fmaf(s, u2, -1.9841270e-4f);
-    s = __builtin_fmaf(s, u2, 8.3333333e-3f);
-    s = __builtin_fmaf(s, u2, -1.6666667e-1f);
-    s = __builtin_fmaf(s * u2, u, u);
-    c = __builtin_fmaf(c, u2, 2.4801587e-5f);
-    c = __builtin_fmaf(c, u2, -1.3888889e-3f);
-    c = __builtin_fmaf(c, u2, 4.1666667e-2f);
-    c = __builtin_fmaf(c, u2, -0.5f);
-    c = __builtin_fmaf(c, u2, 1.0f);
-    const int quad = (int)n;
-    const float x = quad & 1 ? c : s, y = quad & 1 ? s : c;
-    sn[q] = quad & 2 ? -x : x;
-    cs[q] = (quad + 1) & 2 ? -y : y;
-  }
-}
+constexpr int kPNs0 = tr_ns0(kPIn);      // input registers of layer 0 (rows 0..63, row 63 zero)
+constexpr int kPePitch = 65;             // LDS row pitch of the encoding (conflict-free column reads)
 
 // floats of the packed fragments
 __host__ __device__ inline int64_t pe_frag_floats(int depth, int n_out) { return tr_stride(kPIn, kPW, depth, n_out); }
@@ -122,33 +77,39 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
   static_assert(NOUT % 4 == 0 && NOUT <= 32, "output rows in whole 4-row groups of one block");
   constexpr int NSO = NOUT <= 8 ? 4 : 16;  // steps of the output layer's transposed product
   constexpr int NOP = NOUT <= 4 ? 4 : 32;  // delta pitch of the output layer
-  __shared__ __align__(16) uint8_t w_lds[2 * kChunkBytes];
+  // the encodings of the workgroup's samples, then the weight stream's two buffers
+  __shared__ __align__(16) uint8_t lds[4 * 32 * kPePitch * 4];
+  static_assert(sizeof(lds) >= 2 * kChunkBytes, "the weight stream's buffers fit");
   const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int64_t j0 = ((int64_t)blockIdx.x * 4 + wv) * 32;
   const bool any = j0 < n;  // else a wavefront past the end: it keeps the others' barriers
   const int64_t j = j0 + col;
   const bool valid = j < n;
   FragStream fs;
-  fs.start(P, w_lds, chunks);
-  // ---- layer-0 inputs
-  float x0[kPNs0];
-  {
-    float v[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) v[c] = valid ? pts[3 * j + c] : 0.0f;
-    x0[0] = h ? v[2] : v[0];
-    x0[1] = h ? 0.0f : v[1];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      float sn[5], cs[5];
-      pe_bands(v[c], h, sn, cs);
-#pragma unroll
-      for (int q = 0; q < 5; ++q) {
-        x0[2 + 6 * q + c] = sn[q];
-        x0[5 + 6 * q + c] = cs[q];
-      }
-    }
+  fs.start(P, lds, chunks);
+  // ---- positional encoding of the wavefront's 32 samples: [x, sin(2^f x), cos(2^f x)] (f < 10).  sincosf, not a
+  // range reduction shared by the bands (forward of 530k samples: 242 us with that, 261 so): the last bits of the
+  // encoding decide signs of hidden values near zero, and with them gradients.
+  float* E = reinterpret_cast<float*>(lds) + wv * 32 * kPePitch;
+  for (int q = lane; q < 32 * 30; q += 64) {
+    const int smp = q / 30, t = q - 30 * smp, f = t / 3, c = t - 3 * f;
+    const float v = j0 + smp < n ? pts[3 * (j0 + smp) + c] : 0.0f;
+    float sn, cs;
+    sincosf((float)(1 << f) * v, &sn, &cs);
+    E[smp * kPePitch + 3 + 6 * f + c] = sn;
+    E[smp * kPePitch + 6 + 6 * f + c] = cs;
   }
+  for (int q = lane; q < 32 * 4; q += 64) {
+    const int smp = q >> 2, c = q & 3;
+    E[smp * kPePitch + (c < 3 ? c : kPIn)] = (c < 3 && j0 + smp < n) ? pts[3 * (j0 + smp) + c] : 0.0f;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  float x0[kPNs0];
+#pragma unroll
+  for (int s = 0; s < kPNs0; ++s) x0[s] = E[col * kPePitch + tr_row(s, h)];
+  __syncthreads();  // every wavefront has read its encodings
   const int64_t in_rows = pe_rows(n) * kPW;  // floats of one layer's input rows
   const int64_t blk = j0;                    // first sample of this wavefront's block
   if (BWD && any) store_rows<kPW, kPNs0 / 4>(rows + blk * kPW, x0, lane);
@@ -218,19 +179,19 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_mma(const float* __restrict__ 
 
 __global__ __launch_bounds__(kPackThreads) void k_pack_pe(const float* __restrict__ params, float* __restrict__ dst,
                                                           int depth, int n_out) {
-  pack_train_layer(params, dst, kPIn, kPW, depth, blockIdx.x, n_out, [](int row) { return pe_input(row); });
+  pack_train_layer(params, dst, kPIn, kPW, depth, blockIdx.x, n_out);
 }
 
 // dW and db of layer blockIdx.y over split blockIdx.x of the 32-sample blocks (atomics into g_params)
-template <int IP, int OP, int INL, int OUTL, class InOf>
-__device__ void pe_dw_layer(const float* rows, int64_t n, int L, int depth, int n_out, int l, float* g_params,
-                            float* red, InOf in_of) {
+template <int IP, int OP, int INL, int OUTL>
+__device__ __forceinline__ void pe_dw_layer(const float* rows, int64_t n, int L, int depth, int n_out, int l, float* g_params,
+                            float* red) {
   const int64_t blocks = (n + 31) / 32, per = (blocks + gridDim.x - 1) / gridDim.x;
   const int64_t b0 = (int64_t)blockIdx.x * per, b1 = b0 + per < blocks ? b0 + per : blocks;
   if (b0 >= b1) return;  // the whole workgroup
   const int64_t nr = pe_rows(n);
   dw_layer<OP, IP, OUTL, INL>(rows + pe_d_off(l, L, depth, n_out, nr), rows + pe_x_off(l, L, nr), b0, b1,
-                              g_params + pe_param_off(l, L, depth, n_out), red, in_of);
+                              g_params + pe_param_off(l, L, depth, n_out), red);
 }
 
 template <int NOUT>
@@ -240,11 +201,11 @@ __global__ __launch_bounds__(256, 2) void k_pemlp_dw(const float* __restrict__ r
   constexpr int NOP = NOUT <= 4 ? 4 : 32;
   const int l = blockIdx.y;
   if (l == 0) {
-    pe_dw_layer<64, kPW, 63, kPW>(rows, n, L, depth, NOUT, l, g_params, red, [](int i) { return pe_input(i); });
+    pe_dw_layer<64, kPW, 63, kPW>(rows, n, L, depth, NOUT, l, g_params, red);
   } else if (l == depth - 1) {
-    pe_dw_layer<kPW, NOP, kPW, NOUT>(rows, n, L, depth, NOUT, l, g_params, red, [](int i) { return i; });
+    pe_dw_layer<kPW, NOP, kPW, NOUT>(rows, n, L, depth, NOUT, l, g_params, red);
   } else {
-    pe_dw_layer<kPW, kPW, kPW, kPW>(rows, n, L, depth, NOUT, l, g_params, red, [](int i) { return i; });
+    pe_dw_layer<kPW, kPW, kPW, kPW>(rows, n, L, depth, NOUT, l, g_params, red);
   }
 }
 

@@ -1555,9 +1555,9 @@ __global__ __launch_bounds__(256, 2) void k_train_dw(Workspace W, int64_t mlp_st
   float* G = dmlp + (int64_t)tile * mlp_stride + param_w_off(IN, WD, L, l);
   const float* A = W.act + NJ * act_a_off(IN, WD, L, l) + j0 * in_pad_of(IN, WD, l);
   const float* D = W.act + NJ * act_d_off(IN, WD, L, l) + j0 * out_pad_of(WD, L, l);
-  if (l == 0) dw_layer<WD, in_pad_of(IN, WD, 0), WD, IN>(D, A, b0, b1, G, red, [](int i) { return i; });
-  else if (l == L - 1) dw_layer<4, WD, 3, WD>(D, A, b0, b1, G, red, [](int i) { return i; });
-  else dw_layer<WD, WD, WD, WD>(D, A, b0, b1, G, red, [](int i) { return i; });
+  if (l == 0) dw_layer<WD, in_pad_of(IN, WD, 0), WD, IN>(D, A, b0, b1, G, red);
+  else if (l == L - 1) dw_layer<4, WD, 3, WD>(D, A, b0, b1, G, red);
+  else dw_layer<WD, WD, WD, WD>(D, A, b0, b1, G, red);
 }
 
 // The training MLP's matrix helpers (fragment layout, packing, staging) are in train_mma.hpp.
@@ -1565,8 +1565,7 @@ __global__ __launch_bounds__(256, 2) void k_train_dw(Workspace W, int64_t mlp_st
 __global__ __launch_bounds__(kPackThreads) void k_pack_train(const float* __restrict__ src, int64_t src_stride,
                                                              float* __restrict__ dst, int in0, int wd, int L) {
   const int tile = blockIdx.x / L, l = blockIdx.x % L;
-  pack_train_layer(src + (int64_t)tile * src_stride, dst + (int64_t)tile * tr_stride(in0, wd, L, 3), in0, wd, L, l, 3,
-                   [](int row) { return row; });
+  pack_train_layer(src + (int64_t)tile * src_stride, dst + (int64_t)tile * tr_stride(in0, wd, L, 3), in0, wd, L, l, 3);
 }
 
 template <int F, int WD, int L, bool HALF, bool BWD>

@@ -10,14 +10,14 @@ namespace snisr {
 // blocks j0, j0 + dj, ... < j1.  A lane of an operand is a feature and its k slots are records, so both
 // operands come straight from memory in 1 KB loads (no LDS, no barriers), the next half block's loads in
 // flight while the current one is split into its BF16 parts and multiplied.
-// OW / IW: row widths, OUTL / INL: real outputs and inputs; in_of: the input stored at a row.  ONCE: no other
+// OW / IW: row widths, OUTL / INL: real outputs and inputs.  ONCE: no other
 // wavefront reads these blocks, so the loads are non-temporal (1.56 GB of the 530k-sample reflection step: 360 -> 265
 // us with the rows stored so too; blocks that two wavefronts share are 7% slower that way: 2283 -> 2450 us at width 128).
 // With `red` (NA NB 1024 floats of LDS) the workgroup's wavefronts hold the same blocks: they are added there
 // first and only the sums go out.
-template <int OW, int IW, int OUTL, int INL, int NA, int NB, bool ONCE, class InOf>
+template <int OW, int IW, int OUTL, int INL, int NA, int NB, bool ONCE>
 __device__ __forceinline__ void dw_wave(const float* __restrict__ D, const float* __restrict__ A, int64_t j0, int64_t j1,
-                                        int64_t dj, int ob0, int ib0, float* __restrict__ G, InOf in_of, float* red = nullptr) {
+                                        int64_t dj, int ob0, int ib0, float* __restrict__ G, float* red = nullptr) {
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   f32x16 acc[NA][NB];
   float db[NA];
@@ -97,7 +97,7 @@ __device__ __forceinline__ void dw_wave(const float* __restrict__ D, const float
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       if (red && wv) break;
-      const int in = in_of(32 * (ib0 + j) + c);
+      const int in = 32 * (ib0 + j) + c;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int o = 32 * (ob0 + i) + 8 * (r / 4) + 4 * h + (r % 4);
@@ -113,20 +113,20 @@ __device__ __forceinline__ void dw_wave(const float* __restrict__ D, const float
 // dW_l[o][i] += sum_j D_l[j][o] A_l[j][i] and db_l[o] += sum_j D_l[j][o] over the record blocks [j0, j1) of a
 // four-wavefront workgroup.  A layer of at most 2 x 2 blocks gives every wavefront all of them over every
 // fourth record block (red: 4096 floats of LDS); a larger one gives each wavefront a part of the blocks over all records.
-template <int OW, int IW, int OUTL, int INL, class InOf>
+template <int OW, int IW, int OUTL, int INL>
 __device__ __forceinline__ void dw_layer(const float* __restrict__ D, const float* __restrict__ A, int64_t j0, int64_t j1,
-                                         float* __restrict__ G, float* red, InOf in_of) {
+                                         float* __restrict__ G, float* red) {
   constexpr int NOB = (OUTL + 31) / 32, NIB = (INL + 31) / 32;
   const int wv = threadIdx.x >> 6;
   if constexpr (NOB <= 2 && NIB <= 2) {
-    dw_wave<OW, IW, OUTL, INL, NOB, NIB, true>(D, A, j0 + wv, j1, 4, 0, 0, G, in_of, red);
+    dw_wave<OW, IW, OUTL, INL, NOB, NIB, true>(D, A, j0 + wv, j1, 4, 0, 0, G, red);
   } else if constexpr (NOB == 4 && NIB == 4) {
-    dw_wave<OW, IW, OUTL, INL, 2, 2, false>(D, A, j0, j1, 1, 2 * (wv >> 1), 2 * (wv & 1), G, in_of);
+    dw_wave<OW, IW, OUTL, INL, 2, 2, false>(D, A, j0, j1, 1, 2 * (wv >> 1), 2 * (wv & 1), G);
   } else if constexpr (NOB == 4 && NIB == 2) {
-    dw_wave<OW, IW, OUTL, INL, 2, 1, false>(D, A, j0, j1, 1, 2 * (wv >> 1), wv & 1, G, in_of);
+    dw_wave<OW, IW, OUTL, INL, 2, 1, false>(D, A, j0, j1, 1, 2 * (wv >> 1), wv & 1, G);
   } else {
     static_assert(NOB == 1 && NIB == 4, "layer shapes of the training MLPs");
-    dw_wave<OW, IW, OUTL, INL, 1, 2, false>(D, A, j0 + (wv >> 1), j1, 2, 0, 2 * (wv & 1), G, in_of);
+    dw_wave<OW, IW, OUTL, INL, 1, 2, false>(D, A, j0 + (wv >> 1), j1, 2, 0, 2 * (wv & 1), G);
   }
 }
 

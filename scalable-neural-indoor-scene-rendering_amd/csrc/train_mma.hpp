@@ -109,11 +109,9 @@ __device__ __forceinline__ void mma_split(const Split8 (&a)[NA], const Split8 (&
 namespace {
 constexpr int kPackThreads = 512;
 // One workgroup per layer and tile: the layer's forward and transposed fragments and its biases (mlp_params
-// layout: per layer W[out][in], then b[out]; the last layer has nout <= 32 rows).  in_of(row): the input at
-// row `row` of layer 0's products.
-template <class InOf>
+// layout: per layer W[out][in], then b[out]; the last layer has nout <= 32 rows).
 __device__ __forceinline__ void pack_train_layer(const float* __restrict__ P, float* __restrict__ block, int in0, int wd,
-                                                 int L, int l, int nout, InOf in_of) {
+                                                 int L, int l, int nout) {
   for (int m = 0; m < l; ++m) P += (int64_t)((m == 0 ? in0 : wd) + 1) * wd;
   const int in = l == 0 ? in0 : wd, out = l == L - 1 ? nout : wd;
   const int nob = tr_nob(wd, L, l);
@@ -133,8 +131,7 @@ __device__ __forceinline__ void pack_train_layer(const float* __restrict__ P, fl
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int k = tr_row(8 * kc + e, h);
-        int o = bwd ? k : row, i = bwd ? row : k;
-        if (l == 0) i = in_of(i);
+        const int o = bwd ? k : row, i = bwd ? row : k;
         v[e] = kc < nk && o < out && i < in ? P[(int64_t)o * in + i] : 0.0f;
       }
 #pragma unroll

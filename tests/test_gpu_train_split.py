@@ -75,3 +75,17 @@ def test_encoding_ranges_match_fp64(scale):
     p[0][:, :3] = 0.0
     out = mlp(p, 2, 4, 0.0)(x.to(DEV)).detach().cpu().double()
     assert (out - forward64(p, x, 0.0)).abs().max() <= 1e-5
+
+
+def test_points_do_not_depend_on_their_neighbours():
+    p = params(6, 28, 9)
+    x = torch.rand((100, 3), generator=torch.Generator().manual_seed(8)) * 2 - 1
+    m = mlp(p, 6, 28, 0.01)
+    with torch.no_grad():
+        base = m(x.to(DEV))
+        y = x.clone()
+        y[5], y[40] = torch.tensor([5e3, -3e4, 0.1]), float("nan")
+        others = [k for k in range(100) if k not in (5, 40)]
+        assert torch.equal(m(y.to(DEV))[others], base[others])
+        for a, b in ((0, 1), (31, 66), (97, 100)):
+            assert torch.equal(m(x[a:b].to(DEV)), base[a:b])

@@ -196,8 +196,10 @@ __global__ __launch_bounds__(256) void k_query_fwd(const float* __restrict__ vox
 // through LDS, and lane (segment of 8 samples, x side, channel) adds one channel of one x side: the eight
 // lanes of a segment then cover the 32 bytes of two neighbouring corner cells, one transaction instead of
 // eight.  A lane walks its segment in order with a running sum per (y, z) corner pair and adds it only when
-// the cell changes (consecutive samples of a ray often share theirs).  530k samples of a 91x91 patch, one
-// sample per voxel: 327 us with one lane per sample and 4-byte atomics to 64 cells, 79 us now.
+// the cell changes (consecutive samples of a ray often share theirs).  530k samples of 8281 rays in 64^3 voxels, one
+// lane per sample with sums over runs of up to 64 lanes | this: two voxels apart 397 us | 68, one 511 | 95, a
+// quarter 227 | 58, a sixteenth 84 | 36, a 64th 39 | 31; unrelated points 845 | 135; 64k samples in one voxel 152 | 24
+// (221 with every segment adding its own sum).
 constexpr int kQueryPitch = 21;  // floats per staged sample: 8 weights, 8 cells, 4 gradients; odd against bank conflicts
 __global__ __launch_bounds__(256) void k_query_bwd(int D, const float* __restrict__ pts, int64_t n, float3 mc, float vs,
                                                    const float* __restrict__ g_rgb, const float* __restrict__ g_sigma,
@@ -258,8 +260,17 @@ __global__ __launch_bounds__(256) void k_query_bwd(int D, const float* __restric
       }
     }
   }
+  // the runs that are open at the segments' ends; one cell in all eight segments is one add
 #pragma unroll
-  for (int y = 0; y < 4; ++y) flush(cur[y], run[y]);
+  for (int y = 0; y < 4; ++y) {
+    if (__builtin_amdgcn_ballot_w64(cur[y] != __shfl(cur[y], lane & 7)) != 0) {
+      flush(cur[y], run[y]);
+    } else {
+#pragma unroll
+      for (int o = 8; o < 64; o <<= 1) run[y] = run[y] + __shfl_xor(run[y], o);
+      if (seg == 0) flush(cur[y], run[y]);
+    }
+  }
 }
 
 __global__ void k_vox_zero(float4* __restrict__ p, int64_t n) {

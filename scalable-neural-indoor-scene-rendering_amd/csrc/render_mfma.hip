@@ -325,7 +325,7 @@ __device__ __forceinline__ void write_encoding(V3 d, int enc_dtype, uint16_t* ou
 }
 
 // ------------------------------------------------------------------------- march passes
-// A training march pass, every ray on a group of G lanes (march_group_lanes; with one ray per lane the two
+// A training march pass, every ray on a group of G lanes (train_march_lanes; with one ray per lane the two
 // passes took 172 us of the 332 us step of 3,001 rays in one tile, which takes 274 us now)
 template <bool EMIT, int G>  // count the samples, or write their records with the training extras
 __global__ __launch_bounds__(64) void k_march_pass(snisr_scene S, snisr_march_params P, snisr_rays R,
@@ -1812,21 +1812,33 @@ int device_cus() {
 // Lanes per ray of a march over n rays (GroupMarch); 1: one ray per lane (the packet or queue march).
 // A group finds its ray's cells and samples in fewer dependent memory round trips but repeats the
 // walk's arithmetic on each of its lanes, so it pays while the launch has too few wavefronts to cover
-// the waits.  Measured on 256 CUs, whole render in us (27-tile batch | single-tile view | 16-tile room):
-//   n = 5-6k     one lane 386 | 297 | 620     8 lanes 153 | 59 | 113       4 lanes 176 | 68 | 128
-//   n = 20k      one lane 428                 8 lanes 233                  4 lanes 228      2 lanes 287
-//   n = 50-56k   one lane 530 | 258 | 465     4 lanes 384 | 84 | 256       2 lanes 369 | 95 | 253
-//   n = 127k     one lane       233 | 533     4 lanes       124 | 446      2 lanes       115 | 383
-//   n = 200-230k one lane 1087 | 230 | 695    2 lanes 1032 | 146 | 607
-//   n = 400k     one lane 1999                2 lanes 1999
-//   n = 515k     one lane       270 | 1130    2 lanes       236 | 1212
-// Training (no queue march behind it) keeps two lanes at every larger size: 128k rays 4404 -> 4213.
+// the waits.  Whole render on 256 CUs in us, with 8, 4, 2 lanes and 1 (batch of 27 tiles | batch of one tile |
+// single-tile view | 16-tile room):
+//   n = 6-8k     160 183 241 359 | 104 100 124 187 | 61 69 88 130 | 105 116 146 454
+//   n = 15-16k   202 204 262 374 | 139 128 143 207 | 71 76 93 263 | 146 134 174 425
+//   n = 40k      337 301 324 460 | 253 203 196 257 | 98 85 99 230 | 254 207 216 367
+//   n = 56-57k   431 397 371 520 | 328 269 235 290 | 120 100 108 165 | 320 253 239 430
+//   n = 70k      498 441 417 555 | 388 308 273 322 | 133 109 112 222 | 379 298 271 464
+//   n = 90k      611 513 476 606 | 475 360 321 367 | 143 117 117 207 | 462 347 308 430
+//   n = 128k     814 675 685 732 | 649 487 433 471 | 180 140 128 217 | 624 459 393 475
+//   n = 300-346k 1770 1393 1347 1337 | 1431 1026 848 902 | 368 251 203 243 | 1517 1065 867 827
+//   n = 500-522k 2875 2288 2198 2041 | 2372 1669 1330 1386 | 585 386 291 290 | 2295 1584 1288 1133
+// Eight lanes cross four at 8k to 22k rays, four cross two at 30k (one-tile batch), 46-50k (27 tiles, rooms with and
+// without a mesh bound) and 75-88k (single-tile views), two cross the packet march at 250k to over 500k and the queue
+// march, which has no packet's coherence to gain from, at 250k (27 tiles) to over 500k.  The cuts are in the middle of these.
 static int march_group_lanes(int64_t n, bool packets) {
   const int64_t cus = device_cus();
   if (n <= 64 * cus) return 8;
-  if (n <= 224 * cus) return 4;
+  if (n <= 192 * cus) return 4;
   return n <= (packets ? 1024 : 1536) * cus ? 2 : 1;
 }
+
+// The same for the two passes of the training march, which also write the records.  Whole forward in us with 8, 4
+// and 2 lanes (one tile, width 64 | 16 tiles, width 64 | 9 tiles, width 128): 20k rays 150 158 197 | 294 336 464 | 532
+// 557 650, 37k 207 203 240 | 433 436 555 | 852 844 931, 64k 290 279 313 | 630 595 685 | 1374 1331 1402, 128k 504 479
+// 479 | 1126 1075 1092 | 2597 2537 2533, 512k 1796 1688 1677 | 4080 3843 3887 | 9951 9687 9630: eight and four cross at
+// 37k rays in each, and two lanes gain 0.6% at most where they gain.
+static int train_march_lanes(int64_t n) { return n <= 144 * (int64_t)device_cus() ? 8 : 4; }
 
 // resident wavefronts per CU of the queue-fed march (its grid covers the device once), per device
 static int march_queue_waves_per_cu() {
@@ -2167,14 +2179,13 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   SNISR_REQUIRE(ok, SNISR_ERR_SHAPE, "train_forward: unsupported shape F=%d width=%d layers=%d", F, WD, L);
   SNISR_HIP(stage_event(out, 0, st));
   // no ray schedule: sorting arbitrary training rays by (first tile, octant) made the march slower
-  const int lanes = march_group_lanes(n, false) > 2 ? march_group_lanes(n, false) : 2;
+  const int lanes = train_march_lanes(n);
   const dim3 mgrid((unsigned)((n * lanes + 63) / 64));
 #define SNISR_MARCH_PASS(EMIT_, G_)                                                                                   \
   if (lanes == G_)                                                                                                    \
     hipLaunchKernelGGL((k_march_pass<EMIT_, G_>), mgrid, dim3(64), 0, st, *scene, *params, *rays, *out, W);
   SNISR_MARCH_PASS(false, 8)
   SNISR_MARCH_PASS(false, 4)
-  SNISR_MARCH_PASS(false, 2)
   SNISR_LAUNCHED();
   hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nblocks), dim3(kScanBlock), 0, st, W.counts, n, W.offsets,
                      W.block_sums);
@@ -2186,7 +2197,6 @@ int snisr_train_forward(const snisr_scene* scene, const snisr_march_params* para
   SNISR_LAUNCHED();
   SNISR_MARCH_PASS(true, 8)
   SNISR_MARCH_PASS(true, 4)
-  SNISR_MARCH_PASS(true, 2)
 #undef SNISR_MARCH_PASS
   SNISR_LAUNCHED();
   hipLaunchKernelGGL(k_tile_hist, dim3(kSortGrid), dim3(kSortBlock), 0, st, W);

@@ -44,8 +44,9 @@ def test_fp32_render_matches_oracle(oracle_mod, width, n):
         assert np.abs(g["rgb"] - ref["rgb"]).max() <= RGB_TOL
 
 
-# batches on either side of the group sizes: 8 lanes per ray up to 64 rays per CU, 4 up to 224, then 2
-@pytest.mark.parametrize("n", [1, 9, 64, 16384, 16391, 57344, 57351])
+# batches on either side of the group sizes: 8 lanes per ray up to 64 rays per CU, 4 up to 192, then 2; training
+# 8 up to 144, then 4
+@pytest.mark.parametrize("n", [1, 9, 64, 16384, 16391, 36864, 36871, 49152, 49159, 57344, 57351])
 def test_small_batches_match_fp32_path(n):
     from snisr import _native as N
     from snisr import train as TRN

@@ -107,9 +107,10 @@ def test_mfma_deterministic():
 
 
 def test_flattened_march_matches_nested_march_with_bounds_and_visit_lists(oracle_mod):
-    """Arbitrary rays (no image width) take the flattened march loop; camera packets and the FP32
-    path take the nested one.  With per-ray t_hit bounds and precomputed visit lists both loops give
-    the same samples, transmittance, depth and brick lists, and the FP32 oracle agrees."""
+    """A launch of this size and the FP32 render march their rays by groups of lanes, the FP32 march without
+    colours takes the nested per-ray loop (launches above the groups' sizes: test_gpu_large_marches.py).
+    With per-ray t_hit bounds and precomputed visit lists they give the same samples, transmittance, depth and
+    brick lists, and the FP32 oracle agrees."""
     sc, cam, _ = S.config_c1()
     ds = D.DeviceScene(sc, mfma_dtype=N.SNISR_F16)
     dirs = S.camera_rays_np(cam)
@@ -118,10 +119,11 @@ def test_flattened_march_matches_nested_march_with_bounds_and_visit_lists(oracle
     t_hit[::11] = np.inf
     o, d, th = to_dev(cam.origin), to_dev(dirs), to_dev(t_hit)
     vis = D.trace_tiles(ds, o, to_dev(oracle_mod.normalize(dirs)), sc.max_tiles)
-    flat = D.render_mfma(ds, o, d, t_hit=th, visited=vis, brick_cap=16)                      # flattened
-    nested = D.render_fp32(ds, o, d, t_hit=th, visited=vis, image_width=cam.W, brick_cap=16)  # nested
+    flat = D.render_mfma(ds, o, d, t_hit=th, visited=vis, brick_cap=16)
+    plain = D.render_fp32(ds, o, d, t_hit=th, visited=vis, image_width=cam.W, brick_cap=16)
+    nested = D.render_fp32(ds, o, d, t_hit=th, visited=vis, image_width=cam.W, brick_cap=16, rgb=False)
     for k in ("n_samples", "T", "depth", "bricks"):
-        assert torch.equal(flat[k], nested[k]), k
+        assert torch.equal(flat[k], nested[k]) and torch.equal(plain[k], nested[k]), k
     ref = oracle_mod.render(oracle_mod.OracleScene(sc), cam.origin, dirs, t_hit=t_hit, brick_debug=16)
     assert np.array_equal(flat["n_samples"].cpu().numpy(), ref["n_samples"])
     assert np.array_equal(flat["T"].cpu().numpy().view(np.uint32), ref["T"].view(np.uint32))

@@ -1249,10 +1249,11 @@ __device__ __forceinline__ f16x8 interp8_h2<Mfma<SNISR_F16>>(const uint8_t* cons
 // packed weights (~86 KB for width 128 x 4) in LDS once, then its 8 wavefronts process the span's
 // chunks of that tile, each MFMA reading its A fragment from LDS (ds_read_b128, conflict-free).
 // Per layer the accumulators of one 32-row out-block live at a time (32 VGPRs); the layer's input
-// and output activations stay in registers in the B-operand layout.  Two wavefronts share a SIMD: in FP16 the one
-// that is in its MLP goes first (s_setprio), so that the gather's vector instructions fill the matrix unit's
-// shadow instead of delaying its issue (720p frame of 16 tiles 1125 -> 1109 us, two 1080p views 7657 -> 7535; in BF16,
-// whose gather converts more, 4002 -> 4056, so there both keep the default).
+// and output activations stay in registers in the B-operand layout.  Two wavefronts share a SIMD: the one that is
+// in its MLP goes first (s_setprio), so that the gather's vector instructions fill the matrix unit's shadow instead
+// of delaying its issue.  This kernel without and with it, medians of two or three runs that differ by up to 1%
+// (us): 720p frame of 16 tiles 748 | 726 (BF16 728 | 695), two 1080p views 6420 | 6240 (BF16 6497 | 6142),
+// 1.0M unrelated rays BF16 2423 | 2342; the whole frame 1163 | 1147, the views 7976 | 7811.
 template <int F, int WD, int L, bool HALF, int DT>
 __global__ __launch_bounds__(512) void k_mlp_mfma(snisr_scene S, snisr_rays R, RenderWs W) {
   using M = Mfma<DT>;
@@ -1310,7 +1311,7 @@ __global__ __launch_bounds__(512) void k_mlp_mfma(snisr_scene S, snisr_rays R, R
     }
     for (int64_t c = cb0 + wv; c < seg_end; c += nwv) {
       const int32_t nko = c + nwv < seg_end ? W.perm[(c + nwv) * 64 + lane] : -1;
-      if constexpr (DT == SNISR_F16) __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_s_setprio(0);
       // ---- gather: lane (h, s) builds its half of the input column of sample s of both blocks
       int32_t ray[2], valid[2];
       swap_halves(ko >= 0 ? ko / W.cpr : 0, ray[0], ray[1]);
@@ -1396,7 +1397,7 @@ __global__ __launch_bounds__(512) void k_mlp_mfma(snisr_scene S, snisr_rays R, R
       __builtin_amdgcn_sched_barrier(0);
 
       // ---- MLP, A fragments from LDS
-      if constexpr (DT == SNISR_F16) __builtin_amdgcn_s_setprio(3);
+      __builtin_amdgcn_s_setprio(3);
       vec xa[2][NKH], xb[2][NKH];
       {
         const uint8_t* Lp = lds_w + layer_offset(IN, WD, L, 0);
@@ -1540,8 +1541,7 @@ __global__ __launch_bounds__(256) void k_train_comp_bwd(Workspace W, int64_t n, 
 
 // dW and db of one layer of one tile over split blockIdx.x of the tile's record blocks.  Bound by reading the
 // rows (3.3 KB per record).  The previous form staged 32-record tiles through LDS for FP32 products and took
-// 2.99 ms for the 3.04M records of the 16-tile step (3.4 TB/s); this one
-// 2.25 ms (4.4 TB/s).
+// 2.99 ms for the 3.04M records of the 16-tile step (3.4 TB/s); this one 2.13 ms (4.7 TB/s).
 template <int IN, int WD, int L>
 __global__ __launch_bounds__(256, 2) void k_train_dw(Workspace W, int64_t mlp_stride, float* __restrict__ dmlp) {
   __shared__ float red[4096];
@@ -2107,7 +2107,7 @@ int snisr_render_mfma_tuned(const snisr_scene* scene, const snisr_march_params* 
 
 // record splits per (tile, layer) of the weight-gradient reduction: about sixteen workgroups per CU
 // (two are resident at a time), so that the layers' unequal costs even out over many short
-// workgroups (C3: 4 per CU 3.63 ms, 8: 3.05, 16: 2.95, 32: 2.94, 64: 3.01)
+// workgroups (16 tiles, 3.04M records: 4 per CU 2.61 ms, 8: 2.15, 16: 2.13, 32: 2.16, 64: 2.34)
 static int dw_splits(int64_t tile_layers) {
   const int64_t s = 16 * (int64_t)device_cus() / (tile_layers > 0 ? tile_layers : 1);
   return (int)(s < 1 ? 1 : (s > 128 ? 128 : s));

@@ -155,3 +155,21 @@ def test_tile_mlp_units_of_any_scale(shape):
     out3, _ = render_step(sc, Q, o, d, g)
     full = 1.0 - out3["T"]
     assert (out3["rgb"] - torch.stack([full, 0 * full, full], 1)).abs().max() <= 1e-5
+
+
+# Errors of unbiased sums average out over the 22,000 weights: to 1% of their deviation if independent, a quarter
+# leaves room for what they share.  Sums rounded towards one side had a mean of 1.3 to 1.7 deviations here.
+@pytest.mark.parametrize("depth,n_out", [(6, 28), (8, 4)])
+def test_weight_gradients_are_not_biased(depth, n_out):
+    n = 64 * 8281
+    p, x = params(depth, n_out, 1), points(n, 1)
+    g = torch.randn((n, n_out), generator=torch.Generator().manual_seed(2))
+    _, grads = step(p, x, n_out, 1.0, g)
+    q = [t.double().to(DEV).requires_grad_(True) for t in p]
+    x = x.double().to(DEV)
+    h = torch.cat([x] + [f((2.0 ** k) * x) for k in range(10) for f in (torch.sin, torch.cos)], 1)
+    for l in range(depth):
+        h = h @ q[2 * l].T + q[2 * l + 1]
+    h.backward(g.double().to(DEV))
+    err = torch.cat([(a.double() - t.grad.cpu()).reshape(-1) for a, t in zip(grads[::2], q[::2])])
+    assert abs(err.mean()) <= 0.25 * err.std()

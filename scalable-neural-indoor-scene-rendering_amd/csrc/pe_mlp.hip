@@ -300,13 +300,18 @@ int snisr_pemlp_backward(const float* params, const float* points, int64_t n, in
     hipLaunchKernelGGL((k_pemlp_mma<4, true>), grid, dim3(256), 0, st, (const float*)frag, chunks, bias, points, n, (int)depth,
                        slope, nullptr, g_out, rows);
   SNISR_LAUNCHED();
-  // sample splits of the weight-gradient reduction: about four workgroups per CU over all layers,
-  // at least 256 samples and at most 8192 per split
-  const int64_t cus = device_cus();
-  int64_t splits = (4 * cus + depth - 1) / depth;
-  const int64_t lo = (n + 8191) / 8192, hi = (n + 255) / 256;
-  splits = splits < lo ? lo : (splits > hi ? hi : splits);
-  splits = splits < 1 ? 1 : splits;
+  // sample splits of the weight-gradient reduction: one per 1024 samples, but at most the three workgroups per CU, over
+  // all layers, that are resident together, and where the samples give fewer than one per CU, shorter ones down to 384;
+  // at most 8192 samples each.  A workgroup ends with 4096 atomics per block pair into the same gradients, and a
+  // wavefront of a short one has few loads in flight.  k_pemlp_dw with 1, 2, 3, 4 workgroups per CU (us): depth 2, 64k
+  // samples 26 35 35 35, 250k 59 55 67 79, 530k 105 86 93 119; depth 6, 16k 19 22 21 21, 64k 48 47 52 60, 250k 160 140
+  // 133 148, 530k 317 277 246 267; depth 8, 64k 64 56 61 69, 250k 207 159 161 177, 530k 412 316 321 338.
+  const int64_t cus = device_cus(), one = (cus + depth - 1) / depth, few = (n + 383) / 384;
+  int64_t splits = (n + 1023) / 1024;
+  const int64_t least = one < few ? one : few, most = 3 * cus / depth > 1 ? 3 * cus / depth : 1;
+  splits = splits < least ? least : (splits > most ? most : splits);
+  const int64_t longest = (n + 8191) / 8192;
+  splits = splits < longest ? longest : splits;
   const dim3 g((unsigned)splits, (unsigned)depth);
   if (n_out == 28)
     hipLaunchKernelGGL(k_pemlp_dw<28>, g, dim3(256), 0, st, (const float*)rows, n, (int)L, (int)depth, g_params);

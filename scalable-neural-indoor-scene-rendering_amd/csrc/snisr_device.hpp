@@ -483,12 +483,6 @@ struct FlatMarch {
       if (T < P.early_stop) phase = kDone;
     }
   }
-  __device__ __forceinline__ void result(MarchResult& res) const {
-    res.T = T;
-    res.n_samples = nsamp;
-    res.depth = depth;
-    res.n_bricks = nbr;
-  }
 };
 
 // One ray per group of G consecutive lanes (G divides 64).  A wavefront that marches one ray per lane
@@ -670,12 +664,6 @@ struct GroupMarch {
       return mine;
     }
     return false;
-  }
-  __device__ __forceinline__ void result(MarchResult& res) const {
-    res.T = T;
-    res.n_samples = nsamp;
-    res.depth = depth;
-    res.n_bricks = nbr;
   }
 };
 

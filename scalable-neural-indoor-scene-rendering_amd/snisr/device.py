@@ -181,7 +181,7 @@ def _render_outputs(n, device, rgb=True, brick_cap=0):
 
 def render_fp32(ds: DeviceScene, origins, dirs, t_hit=None, visited=None, image_width=0, rgb=True, brick_cap=0,
                 events=None, **march_kw):
-    """One-thread-per-ray FP32 render (snisr_render_fp32)."""
+    """FP32 render, eight lanes per ray (snisr_render_fp32); ``rgb=False`` marches without colours."""
     r = _rays_desc(origins, dirs, t_hit, visited, image_width)
     p = ds.march_params(**march_kw)
     if visited is not None and visited.shape[-1] != p.max_tiles:
